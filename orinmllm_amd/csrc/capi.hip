@@ -361,11 +361,32 @@ int orin_mha_kernel_gpu_pos(const int32_t* pos_ptr, int32_t head_num, int32_t la
                     mha_out, query, score, key_cache, value_cache, stream);
 }
 
-// Causal prefill on the per-row kernel (fp32, or any dtype the MFMA path lacks).
-static int prefill_rows(int32_t start_pos, int32_t seq_len, int32_t head_num, int32_t kv_head_num,
-                        int32_t head_size, int32_t kv_mul, const void* query, void* output,
-                        const void* k, const void* v, int32_t kv_dim, int dtype,
-                        hipStream_t stream) {
+// fp32 causal prefill: the fp32 matrix-core kernel where it is the faster one, else one
+// dot-product workgroup per row and kv head.
+static int prefill_f32(int32_t start_pos, int32_t seq_len, int32_t head_num, int32_t kv_head_num,
+                       int32_t head_size, int32_t kv_mul, const void* query, void* output,
+                       const void* k, const void* v, int32_t kv_dim, hipStream_t stream) {
+  FwdArgs f = {};
+  f.q = query;
+  f.q_tok_stride = (long)head_num * head_size;
+  f.q_head_stride = head_size;
+  f.k = k;
+  f.v = v;
+  f.kv_tok_stride = kv_dim;
+  f.kv_head_stride = head_size;
+  f.o = output;
+  f.o_tok_stride = (long)head_num * head_size;
+  f.o_head_stride = head_size;
+  f.n_q = seq_len;
+  f.start_pos = start_pos;
+  f.causal = 1;
+  f.n_cu = device_cus();
+  f.Hq = head_num;
+  f.Hkv = kv_head_num;
+  f.kv_mul = kv_mul;
+  f.head_size = head_size;
+  f.scale_log2 = resolve_scale(0.f, head_size) * kLog2e;
+  if (fwd_f32_supports(f)) return hip_status(launch_fwd_f32(f, stream));
   DecodeArgs a = decode_defaults();
   a.q = query;
   a.q_row_stride = (long)head_num * head_size;
@@ -385,7 +406,7 @@ static int prefill_rows(int32_t start_pos, int32_t seq_len, int32_t head_num, in
   a.kv_mul = kv_mul;
   a.head_size = head_size;
   a.scale_log2 = resolve_scale(0.f, head_size) * kLog2e;
-  return run_decode(a, dtype, 0, stream);
+  return run_decode(a, kF32, 0, stream);
 }
 
 int orin_batched_mha(int32_t start_pos, int32_t seq_len, int32_t head_num, int32_t layer_index,
@@ -402,9 +423,8 @@ int orin_batched_mha(int32_t start_pos, int32_t seq_len, int32_t head_num, int32
   if (!mha_out || !query || !key_cache || !value_cache) return ORIN_ERR_INVALID_ARG;
   if (!decode_supports(kF32, head_size)) return ORIN_ERR_UNSUPPORTED;
   const long layer_off = (long)layer_index * max_seq_len * kv_dim;
-  return prefill_rows(start_pos, seq_len, head_num, kv_head_num, head_size, kv_mul, query,
-                      mha_out, key_cache + layer_off, value_cache + layer_off, kv_dim, kF32,
-                      (hipStream_t)stream);
+  return prefill_f32(start_pos, seq_len, head_num, kv_head_num, head_size, kv_mul, query, mha_out,
+                     key_cache + layer_off, value_cache + layer_off, kv_dim, (hipStream_t)stream);
 }
 
 // ------------------------------------------------------------------ flash attention
@@ -430,8 +450,8 @@ static int prefill_common(int32_t start_pos, int32_t seq_len, int32_t head_num,
   const bool fused = rope_sin != nullptr;
   if (dtype == kF32) {
     if (fused || !decode_supports(kF32, head_size)) return ORIN_ERR_UNSUPPORTED;
-    return prefill_rows(start_pos, seq_len, head_num, kv_head_num, head_size, kv_mul, query,
-                        output, k, v, kv_dim, kF32, (hipStream_t)stream);
+    return prefill_f32(start_pos, seq_len, head_num, kv_head_num, head_size, kv_mul, query, output,
+                       k, v, kv_dim, (hipStream_t)stream);
   }
   if (!fwd_supports(dtype, head_size)) return ORIN_ERR_UNSUPPORTED;
   FwdArgs a = {};
@@ -792,32 +812,34 @@ static int vision_common(const void* q, const void* k, const void* v, void* outp
   if (cu_seqlens && (n_seqs <= 0 || max_seqlen <= 0)) return ORIN_ERR_INVALID_ARG;
   const float sl2 = resolve_scale(scale, head_dim) * kLog2e;
   const long tok = head_dim, hs = (long)num_tokens * head_dim;
+  FwdArgs f = {};
+  f.q = q;
+  f.q_tok_stride = tok;
+  f.q_head_stride = hs;
+  f.k = k;
+  f.v = v;
+  f.kv_tok_stride = tok;
+  f.kv_head_stride = hs;
+  f.o = output;
+  f.o_tok_stride = (long)num_heads * head_dim;
+  f.o_head_stride = head_dim;
+  f.n_q = num_tokens;
+  f.cu_seqlens = cu_seqlens;
+  f.n_seg = cu_seqlens ? n_seqs : 1;
+  f.max_seqlen = cu_seqlens ? max_seqlen : num_tokens;
+  f.Hq = num_heads;
+  f.Hkv = num_heads;
+  f.kv_mul = 1;
+  f.head_size = head_dim;
+  f.scale_log2 = sl2;
+  f.n_cu = device_cus();
   if (dtype == kF16 || dtype == kBF16) {
     if (!fwd_supports(dtype, head_dim)) return ORIN_ERR_UNSUPPORTED;
-    FwdArgs a = {};
-    a.q = q;
-    a.q_tok_stride = tok;
-    a.q_head_stride = hs;
-    a.k = k;
-    a.v = v;
-    a.kv_tok_stride = tok;
-    a.kv_head_stride = hs;
-    a.o = output;
-    a.o_tok_stride = (long)num_heads * head_dim;
-    a.o_head_stride = head_dim;
-    a.n_q = num_tokens;
-    a.cu_seqlens = cu_seqlens;
-    a.n_seg = cu_seqlens ? n_seqs : 1;
-    a.max_seqlen = cu_seqlens ? max_seqlen : num_tokens;
-    a.Hq = num_heads;
-    a.Hkv = num_heads;
-    a.kv_mul = 1;
-    a.head_size = head_dim;
-    a.scale_log2 = sl2;
-    return hip_status(launch_fwd_varlen(a, dtype, (hipStream_t)stream));
+    return hip_status(launch_fwd_varlen(f, dtype, (hipStream_t)stream));
   }
   if (dtype != kF32) return ORIN_ERR_UNSUPPORTED;
   if (!decode_supports(kF32, head_dim)) return ORIN_ERR_UNSUPPORTED;
+  if (fwd_f32_supports(f)) return hip_status(launch_fwd_f32(f, (hipStream_t)stream));
   DecodeArgs a = decode_defaults();
   a.q = q;
   a.q_row_stride = tok;
