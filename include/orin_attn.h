@@ -140,8 +140,8 @@ int orin_flash_attention_prefill_qk_norm_rope(
  * flash_attention2_decode_cu / flash_attention2_decode_fp16_cu
  * (flash_attention_kernel.cuh:50-63, 84-97, 186-216).  One query row [dim] at
  * position pos over cache rows 0..pos.  Split-KV partials go to the stream's
- * library-owned workspace (see orin_attn_workspace_reserve_stream).  bf16 caches: the
- * weights are split into bf16 hi + lo parts and V is used as stored (bf16's full range).
+ * library-owned workspace (see orin_attn_workspace_reserve_stream); the split size follows
+ * pos alone, so host and device positions give the same bits.  bf16 caches: the weights are split into bf16 hi + lo parts and V is used as stored (bf16's full range).
  */
 int orin_flash_attention_decode(int32_t pos, int32_t head_num, int32_t kv_head_num,
                                 int32_t head_size, int32_t kv_mul, int32_t layer_index,
@@ -168,9 +168,9 @@ int orin_flash_attention_decode_gpu_pos(const int32_t* pos_ptr, int32_t head_num
  * orin_flash_attention_decode_noalloc_max_bytes() bytes (4 MiB) that each GPU holds
  * until the process ends, instead of a library-owned buffer.  It allocates nothing and
  * needs no reserve; the launch and the result equal orin_flash_attention_decode_gpu_pos
- * bit for bit.  A launch whose partials would exceed the array (head_num * splits *
- * (head_size + 2) * 4 bytes; at 32 heads, d 128: a cache of more than 64512 rows) returns
- * ORIN_ERR_WORKSPACE and queues nothing.  Every call on one GPU shares that GPU's array:
+ * bit for bit.  A cache whose 256-token splits' partials would exceed the array (head_num *
+ * splits * (head_size + 2) * 4 bytes; at 32 heads, d 128: a cache of more than 64512 rows)
+ * returns ORIN_ERR_WORKSPACE and queues nothing.  Every call on one GPU shares that GPU's array:
  * calls that overlap in time (other streams, concurrent graph replays) race.  Each call
  * writes every partial it reads, so the array needs no clearing between calls.
  */
@@ -239,12 +239,13 @@ int orin_attn_workspace_release_stream(void* stream);
  * split_tokens: tokens per split (multiple of 64, else ORIN_ERR_INVALID_ARG), 0 =
  * automatic: whole rows (one split per row, no workspace) when batch * kv_head_num is at
  * least the device's CU count, else splits sized from max_context_len alone
- * (orin_attn_decode_split_tokens_for_total uses the batch's total length too).  Launches
- * of whole rows with batch * kv_head_num >= CUs run the matrix-core kernel where it
- * supports the shape (16-bit caches, head_size 64 or 128, at most 16 query heads per kv
- * head); the rest run the dot-product kernel.  Workspace: orin_attn_decode_workspace_size
- * bytes (may be NULL when that is 0).  bf16 caches: V is used as stored (the weights are
- * split into bf16 hi + lo parts), so bf16's full range is kept.
+ * (orin_attn_decode_split_tokens_for_total uses the batch's total length too).  16-bit caches
+ * of head_size 64 or 128 with at most 16 query heads per kv head run on the matrix cores, the
+ * rest on the dot-product kernel, whose automatic splits may be larger
+ * (orin_attn_decode_split_tokens returns the matrix-core choice where the head counts allow
+ * it).  Workspace: orin_attn_decode_workspace_size bytes (may be NULL when that is 0).  bf16
+ * caches: V is used as stored (the weights are split into bf16 hi + lo parts), so bf16's full
+ * range is kept.
  */
 size_t orin_attn_decode_workspace_size(int32_t batch, int32_t head_num, int32_t kv_head_num,
                                        int32_t head_size, int32_t max_context_len,

@@ -5,6 +5,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -36,16 +37,15 @@ constexpr int kMaxSplits = 1024;
 
 int device_cus();
 
-// Tokens per split for a decode launch with `base_blocks` (row, kv head, head group)
-// units and rows of up to max_len tokens.
+// Tokens per split for a decode launch with `base_blocks` (row, kv head, head group) units and
+// rows of up to max_len tokens on the dot-product kernel.
 //  * At least one unit per CU: whole rows (one split), so no partials and no merge launch.
 //    Each unit is then one workgroup that streams its row (for 16-bit caches at head size
 //    64 / 128 on the matrix-core kernel).  Batch 32 x 8 kv heads (fp16, d 128): every
 //    length 4096 0.76-0.77 of HBM against 0.66 with 320-token splits; lengths U[512, 4096]
 //    0.64 against 0.62-0.63 with 320-token splits plus their merge.
 //  * Fewer units: aims at ~3328 workgroups (13 per CU, i.e. about 3.25 rounds of the 4
-//    resident per CU; measured best on the batch-32 paged decode) with at least 256 tokens
-//    (one 64-token tile per wave) per split.
+//    resident per CU) with at least 256 tokens (one 64-token tile per wave) per split.
 int auto_split_tokens(long base_blocks, int max_len) {
   if (max_len <= 0) return 256;
   if (base_blocks >= device_cus()) return round_up(max_len, 64);
@@ -54,6 +54,27 @@ int auto_split_tokens(long base_blocks, int max_len) {
   if (splits < 1) splits = 1;
   int st = round_up((max_len + splits - 1) / splits, 64);
   if (st < 256) st = 256;
+  if (st >= max_len) st = round_up(max_len, 64);
+  while ((max_len + st - 1) / st > kMaxSplits) st *= 2;
+  return st;
+}
+
+// The same for the matrix-core split kernel with `units` (row, kv head) pairs, fewer than CUs:
+// a workgroup per CU while that leaves few tokens to a split (their round trips bound it), then
+// 256 tokens.  us at splits of 64 / 128 / 192 / 256 / 320 / 384 / 512 (KV not in cache from the
+// third line on):
+//   batch 13, 12/2, bf16, U[227, 454]       8.1 /  8.9 /    - / 10.6 /    - / 12.0 / 10.3  (here 64)
+//   one row of 4096, 32/8 heads, fp16       9.7 /  8.9 /    - / 10.7 /    - / 12.5 / 14.4  (128)
+//   batch 24, 32/8, fp16, U[300, 1200]        - / 21.6 / 21.8 / 20.2 / 25.1 / 26.6 / 22.7  (256)
+//   batch 24, 32/8, fp16, U[512, 4096]        - / 49.9 / 46.3 / 45.5 / 45.3 / 44.6 / 46.3  (256)
+//   batch 5, 28/4, bf16, U[2048, 16000]       - / 32.2 / 30.2 / 30.5 / 29.2 / 28.9 / 30.8  (256)
+//   batch 64, 12/2, bf16, U[300, 4000]        - / 39.7 / 34.6 / 39.9 / 35.2 / 35.8 / 42.0  (256)
+int auto_split_tokens_mfma(long units, int max_len) {
+  if (max_len <= 0) return 256;
+  const long cus = device_cus();
+  if (units >= cus) return round_up(max_len, 64);
+  const long per_cu = units * max_len / cus;
+  int st = per_cu <= 64 ? 64 : per_cu <= 192 ? 128 : 256;
   if (st >= max_len) st = round_up(max_len, 64);
   while ((max_len + st - 1) / st > kMaxSplits) st *= 2;
   return st;
@@ -183,6 +204,7 @@ int device_cus() {
 
 DecodeArgs decode_defaults() {
   DecodeArgs a = {};
+  a.dyn_splits_log2 = -1;
   a.max_splits = 1;
   a.split_tokens = 1 << 30;
   return a;
@@ -200,22 +222,37 @@ int kuiper_decode_split(int head_num, int kv_head_num, int head_size, int max_le
   return st;
 }
 
+// The matrix-core split kernel's single-sequence decode sizes its splits from the row's length
+// (single_row_split_tokens): log2 of the most splits it may use, a workgroup per CU at most 64
+// deep, and no more than the fixed array of the entry point that allocates nothing holds, so
+// that both give the same bits.
+constexpr size_t kNoAllocScratchBytes = 4u << 20;
+int single_row_splits_log2(int head_num, int kv_head_num, int head_size) {
+  int n = 6;
+  while (n > 0 && ((1 << n) * kv_head_num > device_cus() ||
+                   ws_bytes(1, head_num, head_size, 1 << n) > kNoAllocScratchBytes))
+    --n;
+  return n;
+}
+// Splits of a launch that covers rows of up to max_len tokens.
+int single_row_max_splits(int max_len, int splits_log2) {
+  if (max_len <= 128) return 1;
+  return std::min((max_len + 31) / 32, 1 << splits_log2);
+}
+
 // max_len: the longest row the launch must cover (0 = rows are single-split by
-// construction).  Rows are clamped to max_splits * split_tokens tokens.
+// construction).  Rows are clamped to max_splits * split_tokens tokens.  a.dyn_splits_log2 >= 0:
+// the caller set a.max_splits.
 int run_decode(DecodeArgs& a, int dtype, int max_len, hipStream_t stream) {
-  a.max_splits = n_splits(max_len, a.split_tokens);
+  if (a.dyn_splits_log2 < 0) a.max_splits = n_splits(max_len, a.split_tokens);
   if (a.max_splits <= 1) a.max_splits = 1;
   // Dot-product kernel: 16-wave workgroups (where the shape fits) when each (row, kv head,
   // head group) is one split, or when the launch has no more workgroups than the device has
   // CUs: 4-wave workgroups would then leave most wave slots idle.
   const long units = (long)a.n_rows * a.Hkv * (a.kv_mul / decode_heads_per_block(a.kv_mul));
   a.wide = a.max_splits == 1 || units * a.max_splits <= device_cus();
-  // Whole rows of a launch with a (row, kv head) per CU or more: matrix-core kernel.  The
-  // single-sequence (kuiper) decode never qualifies, so its result does not depend on
-  // whether the launch was sized for the position or for the cache capacity.
-  a.mfma = a.max_splits == 1 && (long)a.n_rows * a.Hkv >= device_cus();
   a.len_cap = max_len > 0 ? max_len : (1 << 30);
-  return hip_status(launch_decode(a, dtype, stream));
+  return hip_status(launch_decode(a, device_cus(), dtype, stream));
 }
 
 }  // namespace
@@ -521,7 +558,6 @@ int orin_flash_attention_prefill_qk_norm_rope(
 // entry point never allocates.  In host code `scratch` names a host-side stand-in, not
 // device memory: its device address is looked up once per device (noalloc_scratch) and
 // only that address is passed to kernels.
-static constexpr size_t kNoAllocScratchBytes = 4u << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 static std::mutex g_scratch_mu;
@@ -562,15 +598,27 @@ static int flash_decode_common(int32_t pos, const int32_t* pos_ptr, int32_t head
   const int max_len = pos_ptr ? max_seq_len : pos + 1;
   DecodeArgs a = decode_defaults();
   a.split_tokens = kuiper_decode_split(head_num, kv_head_num, head_size, max_len, 0, false);
-  const int splits = n_splits(max_len, a.split_tokens);
-  const size_t need = ws_bytes(1, head_num, head_size, splits);
+  const size_t fixed_need = ws_bytes(1, head_num, head_size, n_splits(max_len, a.split_tokens));
+  size_t need = fixed_need;
+  if (decode_mfma_supports(dtype, head_size, kv_mul)) {
+    a.dyn_splits_log2 = single_row_splits_log2(head_num, kv_head_num, head_size);
+    a.max_splits = single_row_max_splits(max_len, a.dyn_splits_log2);
+    need = ws_bytes(1, head_num, head_size, a.max_splits);
+  }
   void* ws = nullptr;
   int st;
   if (noalloc) {
-    if (need > kNoAllocScratchBytes) return ORIN_ERR_WORKSPACE;
+    // The documented limit is that of the fixed splits (the largest either kernel forms).
+    if (fixed_need > kNoAllocScratchBytes) return ORIN_ERR_WORKSPACE;
     st = noalloc_scratch(&ws);
   } else {
     st = library_workspace(kWsDecode, (hipStream_t)stream, need, &ws);
+    if (st == ORIN_ERR_WORKSPACE && need > fixed_need) {
+      // A capturing stream whose buffer holds only the fixed 256-token splits' partials (none
+      // for caches of up to 256 rows): use those.
+      a.dyn_splits_log2 = -1;
+      st = library_workspace(kWsDecode, (hipStream_t)stream, fixed_need, &ws);
+    }
   }
   if (st != ORIN_OK) return st;
   const size_t layer_off = (size_t)layer_index * max_seq_len * kv_dim * elem_size(dtype);
@@ -641,8 +689,10 @@ size_t orin_flash_attention_decode_workspace_size(int32_t head_num, int32_t head
   if (head_num <= 0 || head_size <= 0 || max_seq_len <= 0) return 0;
   // Worst case over kv_head_num: the split size shrinks as the unit count drops,
   // so size for kv_head_num = 1.
+  // The matrix-core kernel forms at most 64 splits of at least 32 tokens.
   const int st = auto_split_tokens(decode_base_blocks(1, 1, 1), max_seq_len);
-  return ws_bytes(1, head_num, head_size, n_splits(max_seq_len, st));
+  return ws_bytes(1, head_num, head_size,
+                  std::max(n_splits(max_seq_len, st), single_row_max_splits(max_seq_len, 6)));
 }
 
 size_t orin_flash_attention_prefill_workspace_size(int32_t start_pos, int32_t seq_len,
@@ -668,11 +718,19 @@ size_t orin_flash_attention_prefill_workspace_size(int32_t start_pos, int32_t se
 
 // ------------------------------------------------------------------ batched decode
 
+// The automatic split of a batched decode: `matrix` = the launch runs on the matrix-core kernels.
+static int batched_auto_split(int batch, int head_num, int kv_head_num, int max_len, bool matrix) {
+  const long base = decode_base_blocks(batch, head_num, kv_head_num);
+  return matrix && base < device_cus() ? auto_split_tokens_mfma((long)batch * kv_head_num, max_len)
+                                       : auto_split_tokens(base, max_len);
+}
+
 int32_t orin_attn_decode_split_tokens(int32_t batch, int32_t head_num, int32_t kv_head_num,
                                       int32_t max_context_len, int32_t split_tokens) {
   if (split_tokens > 0) return split_tokens;
   if (batch <= 0 || kv_head_num <= 0 || head_num % kv_head_num) return 0;
-  return auto_split_tokens(decode_base_blocks(batch, head_num, kv_head_num), max_context_len);
+  return batched_auto_split(batch, head_num, kv_head_num, max_context_len,
+                            decode_mfma_supports(kF16, 128, head_num / kv_head_num));
 }
 
 int32_t orin_attn_decode_split_tokens_for_total(int32_t batch, int32_t head_num,
@@ -704,7 +762,13 @@ size_t orin_attn_decode_workspace_size(int32_t batch, int32_t head_num, int32_t 
   const int st =
       orin_attn_decode_split_tokens(batch, head_num, kv_head_num, max_context_len, split_tokens);
   if (st <= 0 || head_size <= 0) return 0;
-  return ws_bytes(batch, head_num, head_size, n_splits(max_context_len, st));
+  int splits = n_splits(max_context_len, st);
+  // The element type is not known here: automatic splits must fit either kernel's choice.
+  if (split_tokens <= 0)
+    splits = std::max(splits, n_splits(max_context_len,
+                                       batched_auto_split(batch, head_num, kv_head_num,
+                                                          max_context_len, false)));
+  return ws_bytes(batch, head_num, head_size, splits);
 }
 
 static int batched_decode(const void* query, const void* k, const void* v, void* out,
@@ -729,11 +793,20 @@ static int batched_decode(const void* query, const void* k, const void* v, void*
     if ((block_size & (block_size - 1)) || block_size < 8) return ORIN_ERR_UNSUPPORTED;
     while ((1 << bs_log2) < block_size) ++bs_log2;
   }
-  const int st =
-      orin_attn_decode_split_tokens(batch, head_num, kv_head_num, max_context_len, split_tokens);
+  const auto ws_need = [&](int st) {
+    return ws_bytes(batch, head_num, head_size, n_splits(max_context_len, st));
+  };
+  const size_t ws_have = workspace ? workspace_bytes : 0;
+  int st = split_tokens;
+  if (st == 0) {
+    const bool matrix = decode_mfma_supports(dtype, head_size, head_num / kv_head_num);
+    st = batched_auto_split(batch, head_num, kv_head_num, max_context_len, matrix);
+    // A workspace sized for the dot-product kernel's splits is enough for this launch too.
+    if (matrix && ws_need(st) > ws_have)
+      st = batched_auto_split(batch, head_num, kv_head_num, max_context_len, false);
+  }
   if (n_splits(max_context_len, st) > kMaxSplits) return ORIN_ERR_INVALID_ARG;
-  const size_t need = ws_bytes(batch, head_num, head_size, n_splits(max_context_len, st));
-  if (need > 0 && (!workspace || workspace_bytes < need)) return ORIN_ERR_WORKSPACE;
+  if (ws_need(st) > ws_have) return ORIN_ERR_WORKSPACE;
   DecodeArgs a = decode_defaults();
   a.split_tokens = st;
   a.q = query;

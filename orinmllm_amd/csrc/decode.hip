@@ -1,9 +1,10 @@
-// Split-KV decode attention for gfx950.
+// Split-KV decode attention for gfx950 on dot products, and the merge of split partials.
 //
 // Replaces the reference's single-query attention kernels
 // (kuiper/source/op/kernels/cuda/mha_kernel.cu:162-338,
 //  flash_attention_kernel.cu:205-535 and :966-1175,
-//  flash_attention2_kernel.cu:409-816) with one design:
+//  flash_attention2_kernel.cu:409-816) for the caches the matrix-core kernels
+// (decode_mfma.hip) do not take: fp32, head size 256, more than 16 query heads per kv head.
 //
 //  * A workgroup (4 waves) owns one (row, kv head, head group, split): it reads that
 //    split's K/V once and serves the G query heads that share the kv head (GQA), so KV
@@ -461,94 +462,118 @@ decode_split_kernel(DecodeArgs a) {
     if (direct) {
       out[(long)(h0 + g) * a.o_head_stride + dd] = from_f32<T>(o / L);
     } else {
-      float* p = a.ws + ((((long)row * a.Hq + h0 + g) * a.max_splits + split) * (D + 2));
-      p[dd] = o;
+      const long pi = ((long)row * a.Hq + h0 + g) * a.max_splits + split;
+      a.ws[pi * D + dd] = o;
       if (dd == 0) {
-        p[D] = M;
-        p[D + 1] = L;
+        float* ml = a.ws + (long)a.n_rows * a.Hq * a.max_splits * D + pi * 2;
+        ml[0] = M;
+        ml[1] = L;
       }
     }
   }
 }
 
-// Merge split partials of every (row, head) whose row needed more than one split.
-// One wave per (row, head): the splits' (m, l) are staged in LDS by the lanes in
-// parallel, then lane l forms outputs [l * D/64, (l + 1) * D/64) with the acc loads of
-// eight splits in flight at a time.
+// Merge the split partials of every (row, head) whose row needed more than one split: acc rows
+// [n_rows, Hq, max_splits][D], then (m, l) pairs.  A workgroup of 256 threads per (row, head):
+// D / 4 threads form a group that owns 4 dimensions each of every NG-th split, and the groups
+// merge through LDS.  The kernel is a chain of memory round trips (the partials come from other
+// XCDs' workgroups), so the first kUp splits of every group are requested before the row's
+// length is known: slots past the row's splits hold stale partials of the workspace, read and
+// not used.
+constexpr int kCombineThreads = 256;
 template <typename T, int D>
-__global__ void __launch_bounds__(64) decode_combine_kernel(DecodeArgs a) {
-  constexpr int EPL = D / kWave;
+__global__ void __launch_bounds__(kCombineThreads) decode_combine_kernel(DecodeArgs a) {
+  constexpr int LPG = D / 4;                  // threads per group
+  constexpr int NG = kCombineThreads / LPG;   // groups
+  constexpr int kUp = 4;
   const int h = blockIdx.x % a.Hq;
   const int row = blockIdx.x / a.Hq;
+  const int j = threadIdx.x % LPG, grp = threadIdx.x / LPG;
+  const long p0 = ((long)row * a.Hq + h) * a.max_splits;
+  const float* acc = a.ws + p0 * D + 4 * j;
+  const float* ml = a.ws + (long)a.n_rows * a.Hq * a.max_splits * D + p0 * 2;
+  f32x4 x[kUp];
+  float m[kUp], l[kUp];
+  const int top = a.max_splits - 1;
+#pragma unroll
+  for (int u = 0; u < kUp; ++u) {
+    const int sp = min(grp + u * NG, top);
+    m[u] = ml[sp * 2];
+    l[u] = ml[sp * 2 + 1];
+    x[u] = *reinterpret_cast<const f32x4*>(acc + (long)sp * D);
+  }
   const int len = row_len(a, row);
   if (len > a.len_cap) return;  // the split kernel wrote NaN
-  const int nsplit = len > 0 ? (len + a.split_tokens - 1) / a.split_tokens : 0;
+  const int st = row_split_tokens(a, len);
+  const int nsplit = len > 0 ? (len + st - 1) / st : 0;
   if (nsplit <= 1) return;
-  const float* ph = a.ws + ((long)row * a.Hq + h) * a.max_splits * (D + 2);
-  const float* pl = ph + threadIdx.x * EPL;
-  // The first kFirst partial rows are loaded before (m, l), so both memory round trips
-  // overlap instead of running one after the other.
-  constexpr int kFirst = 16;
-  float x0[kFirst][EPL];
+  float M = -INFINITY, L = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = grp;;) {
+    float Mn = M;
 #pragma unroll
-  for (int u = 0; u < kFirst; ++u)
-    if (u < nsplit)
+    for (int u = 0; u < kUp; ++u) {
+      if (s0 + u * NG >= nsplit) m[u] = -INFINITY;
+      Mn = fmaxf(Mn, m[u]);
+    }
+    const float Mu = Mn == -INFINITY ? 0.f : Mn;
+    const float r = fast_exp2(M - Mu);
+    M = Mn;
+    L *= r;
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) x0[u][e] = pl[u * (D + 2) + e];
-  __shared__ float s_m[kMaxCombineSplits], s_l[kMaxCombineSplits];
-  float M = -INFINITY;
-  for (int sp = threadIdx.x; sp < nsplit; sp += kWave) {
-    const float m = ph[sp * (D + 2) + D];
-    s_m[sp] = m;
-    s_l[sp] = ph[sp * (D + 2) + D + 1];
-    M = fmaxf(M, m);
+    for (int e = 0; e < 4; ++e) o[e] *= r;
+#pragma unroll
+    for (int u = 0; u < kUp; ++u)
+      if (s0 + u * NG < nsplit) {
+        const float f = fast_exp2(m[u] - Mu);
+        L = __builtin_fmaf(f, l[u], L);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(f, x[u][e], o[e]);
+      }
+    s0 += kUp * NG;
+    if (s0 - grp >= nsplit) break;
+#pragma unroll
+    for (int u = 0; u < kUp; ++u) {
+      const int sp = min(s0 + u * NG, top);
+      m[u] = ml[sp * 2];
+      l[u] = ml[sp * 2 + 1];
+      x[u] = *reinterpret_cast<const f32x4*>(acc + (long)sp * D);
+    }
   }
-#pragma unroll
-  for (int mask = 32; mask >= 1; mask >>= 1) M = fmaxf(M, shfl_xor_f(M, mask));
+  __shared__ f32x4 s_o[NG][LPG];
+  __shared__ float s_ml[NG][2];
+  s_o[grp][j] = o;
+  if (j == 0) {
+    s_ml[grp][0] = M;
+    s_ml[grp][1] = L;
+  }
   __syncthreads();
-  float L = 0.f, o[EPL];
+  if (grp) return;
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) o[e] = 0.f;
+  for (int g = 0; g < NG; ++g) M = fmaxf(M, s_ml[g][0]);
+  L = 0.f;
+  o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int u = 0; u < kFirst; ++u)
-    if (u < nsplit) {
-      const float f = fast_exp2(s_m[u] - M);
-      L = __builtin_fmaf(f, s_l[u], L);
+  for (int g = 0; g < NG; ++g) {
+    const float f = fast_exp2(s_ml[g][0] - M);
+    L = __builtin_fmaf(f, s_ml[g][1], L);
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) o[e] = __builtin_fmaf(f, x0[u][e], o[e]);
-    }
-  int sp = kFirst;
-  for (; sp + 8 <= nsplit; sp += 8) {
-    float x[8][EPL];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) x[u][e] = pl[(sp + u) * (D + 2) + e];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const float f = fast_exp2(s_m[sp + u] - M);
-      L = __builtin_fmaf(f, s_l[sp + u], L);
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) o[e] = __builtin_fmaf(f, x[u][e], o[e]);
-    }
-  }
-  for (; sp < nsplit; ++sp) {
-    const float f = fast_exp2(s_m[sp] - M);
-    L = __builtin_fmaf(f, s_l[sp], L);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) o[e] = __builtin_fmaf(f, pl[sp * (D + 2) + e], o[e]);
+    for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(f, s_o[g][j][e], o[e]);
   }
   const float inv = 1.f / L;
-  T* out = reinterpret_cast<T*>(a.o) + (long)row * a.o_row_stride + (long)h * a.o_head_stride;
+  T* out = reinterpret_cast<T*>(a.o) + (long)row * a.o_row_stride + (long)h * a.o_head_stride + 4 * j;
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  t4 y;
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) out[threadIdx.x * EPL + e] = from_f32<T>(o[e] * inv);
+  for (int e = 0; e < 4; ++e) y[e] = from_f32<T>(o[e] * inv);
+  *reinterpret_cast<t4*>(out) = y;
 }
 
 template <typename T, int D>
 hipError_t launch_combine(const DecodeArgs& a, hipStream_t stream) {
   if (a.max_splits > 1)
-    hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)(a.n_rows * a.Hq)), dim3(64),
-                       0, stream, a);
+    hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)(a.n_rows * a.Hq)),
+                       dim3(kCombineThreads), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -614,12 +639,14 @@ bool decode_supports(int dtype, int head_size) {
          (head_size == 64 || head_size == 128 || head_size == 256);
 }
 
-hipError_t launch_decode(const DecodeArgs& a, int dtype, hipStream_t stream) {
-  // Launches of whole rows that fill the device go to the matrix-core kernel, which streams
-  // a row faster per CU; split launches stay on the dot-product kernel, whose small
-  // workgroups balance ragged rows better.
-  if (a.mfma && a.max_splits == 1 && decode_mfma_supports(dtype, a.head_size, a.kv_mul))
-    return launch_decode_mfma(a, dtype, stream);
+hipError_t launch_decode(const DecodeArgs& a, int n_cu, int dtype, hipStream_t stream) {
+  if (decode_mfma_supports(dtype, a.head_size, a.kv_mul)) {
+    const hipError_t e = launch_decode_mfma(a, n_cu, dtype, stream);
+    if (e != hipSuccess || a.max_splits == 1) return e;
+    if (a.head_size == 64)
+      return dtype == kF16 ? launch_combine<f16, 64>(a, stream) : launch_combine<bf16, 64>(a, stream);
+    return dtype == kF16 ? launch_combine<f16, 128>(a, stream) : launch_combine<bf16, 128>(a, stream);
+  }
   const int G = decode_heads_per_block(a.kv_mul);
   switch (dtype) {
     case kF32: return launch_decode_d<float>(a, G, stream);

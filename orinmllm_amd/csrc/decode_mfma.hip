@@ -5,20 +5,20 @@
 // plus the batched / paged decode) for fp16 / bf16 K and V, head sizes 64 and 128, and up
 // to 16 query heads per kv head.
 //
-// Why a second decode kernel.  launch_decode sends it the launches whose rows are not split
-// (one workgroup per (row, kv head)), where a single CU must stream a whole row: here the
-// two contractions run on the matrix cores, the VALU work per 32-token tile is the softmax
-// of 8 scores per lane, and the loads are whole coalesced rows.  Measured on the batch-32
-// paged decode (fp16, d 128, lengths U[512, 4096]), whole rows: this kernel 0.64 of HBM,
-// the dot-product kernel's 16-wave workgroups 0.59; a copy of this kernel with the
-// arithmetic removed 0.67, so what remains is the rate at which one CU streams a row
-// (~36 GB/s), not its arithmetic.  Split launches stay on the dot-product kernel (this one
-// with 1024-token splits and the merge launch: 0.53-0.54).
+// Two kernels: whole rows (first below) and split rows (further down).
 //
-// Work decomposition.  A workgroup of 4 waves owns one (row, kv head, split) and all G
-// query heads of that kv head (G <= 16, padded to 16 columns).  Wave w takes the 32-token
-// tiles w, w + 4, ... of the split, with its own online-softmax state; the waves are merged
-// once through LDS at the end.  Per tile:
+// Whole rows.  Launches with a (row, kv head) per CU or more and one split per row, where a
+// single CU must stream a whole row: the two contractions run on the matrix cores, the VALU
+// work per 32-token tile is the softmax of 8 scores per lane, and the loads are whole coalesced
+// rows.  Measured on the batch-32 paged decode (fp16, d 128, lengths U[512, 4096]): 0.64 of
+// HBM, the dot-product kernel's 16-wave workgroups 0.59; a copy of this kernel with the
+// arithmetic removed 0.67, so what remains is the rate at which one CU streams a row
+// (~36 GB/s), not its arithmetic.
+//
+// Work decomposition.  A workgroup of 4 waves owns one (row, kv head) and all G query heads of
+// that kv head (G <= 16, padded to 16 columns).  Wave w takes the 32-token tiles w, w + 4, ...
+// of the row, with its own online-softmax state; the waves are merged once through LDS at the
+// end.  Per tile:
 //   S^T[32 x 16] = K[32 x D] . Q^T[D x 16]        2 x D/32  v_mfma_f32_16x16x32
 //   O^T[D x 16] += V^T[D x 32] . P^T[32 x 16]     D/16      v_mfma_f32_16x16x32 (fp16)
 //                                                 2 x D/16  (bf16: P = hi + lo, both bf16)
@@ -89,28 +89,20 @@ __global__ void __launch_bounds__(kMThreads) decode_mfma_kernel(DecodeArgs a) {
   // reuses the space.
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
-  int bid = blockIdx.x;
-  const int kvh = bid % a.Hkv;
-  bid /= a.Hkv;
-  const int split = bid % a.max_splits;
-  const int row = bid / a.max_splits;
+  const int kvh = (int)blockIdx.x % a.Hkv;
+  const int row = (int)blockIdx.x / a.Hkv;
   const int G = a.kv_mul;
   const int h0 = kvh * G;
 
   const int len = row_len(a, row);
-  const int nsplit = len > 0 ? (len + a.split_tokens - 1) / a.split_tokens : 0;
   T* out = reinterpret_cast<T*>(a.o) + (long)row * a.o_row_stride;
   if (len > a.len_cap || len <= 0) {  // past the launch bound: NaN; empty row: zeros
-    if (split == 0) {
-      const float fill = len > 0 ? __builtin_nanf("") : 0.f;
-      for (int i = threadIdx.x; i < G * D; i += kMThreads)
-        out[(long)(h0 + i / D) * a.o_head_stride + i % D] = from_f32<T>(fill);
-    }
+    const float fill = len > 0 ? __builtin_nanf("") : 0.f;
+    for (int i = threadIdx.x; i < G * D; i += kMThreads)
+      out[(long)(h0 + i / D) * a.o_head_stride + i % D] = from_f32<T>(fill);
     return;
   }
-  if (split >= nsplit) return;
-  const int s0 = split * a.split_tokens;
-  const int s1 = min(s0 + a.split_tokens, len);
+  const int s1 = len;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -130,9 +122,7 @@ __global__ void __launch_bounds__(kMThreads) decode_mfma_kernel(DecodeArgs a) {
     bmask = (1 << a.bs_log2) - 1;
   } else {
     // contiguous: token t of the row is at element base + t * kv_tok_stride
-    const long base = a.cu_seqlens
-                          ? (long)a.cu_seqlens[find_segment(a.cu_seqlens, a.n_seg, row)] * a.kv_tok_stride
-                          : (long)row * a.kv_row_stride;
+    const long base = (long)row * a.kv_row_stride;
     kbase += base * (long)sizeof(T);
     vbase += base * (long)sizeof(T);
   }
@@ -316,7 +306,7 @@ __global__ void __launch_bounds__(kMThreads) decode_mfma_kernel(DecodeArgs a) {
   // ahead of the loads that use them.  Loads are issued unconditionally, two buffers deep,
   // so that every wait before a tile's use is the same vmcnt: past the end of the split
   // every lane's token clamps to s1 - 1 and the tile reads one 256-byte row.
-  const int tw0 = s0 + wave * kMTile;
+  const int tw0 = wave * kMTile;
   const int n_w = tw0 < s1 ? (s1 - tw0 + step - 1) / step : 0;
   if (n_w > 0) {
     Regs ra, rb;
@@ -360,7 +350,6 @@ __global__ void __launch_bounds__(kMThreads) decode_mfma_kernel(DecodeArgs a) {
       for (int i = 0; i < 4; ++i) s_o[(wave * G + n) * D + 16 * t + 4 * g + i] = oacc[t][i] * f;
   }
   __syncthreads();
-  const bool direct = nsplit == 1;
   for (int i = threadIdx.x; i < G * D; i += kMThreads) {
     const int hn = i / D, dd = i % D;
     float Mh = -INFINITY;
@@ -373,61 +362,384 @@ __global__ void __launch_bounds__(kMThreads) decode_mfma_kernel(DecodeArgs a) {
       L += mw == -INFINITY ? 0.f : fast_exp2(mw - Mh) * s_l[w * 16 + hn];
       o += s_o[(w * G + hn) * D + dd];
     }
-    if (direct) {
-      out[(long)(h0 + hn) * a.o_head_stride + dd] = from_f32<T>(o / L);
-    } else {
-      float* pp = a.ws + ((((long)row * a.Hq + h0 + hn) * a.max_splits + split) * (D + 2));
-      pp[dd] = o;
-      if (dd == 0) {
-        pp[D] = Mh;
-        pp[D + 1] = L;
-      }
-    }
+    out[(long)(h0 + hn) * a.o_head_stride + dd] = from_f32<T>(o / L);
   }
 }
 
-template <typename T, int D, bool PAGED>
-hipError_t launch_tp(const DecodeArgs& a, hipStream_t stream) {
-  const long blocks = (long)a.n_rows * a.Hkv * a.max_splits;
-  const size_t lds = decode_mfma_lds_bytes(D);
-  const void* fn = (const void*)decode_mfma_kernel<T, D, PAGED>;
-  // More than 64 KB of dynamic LDS must be granted per kernel (once per device).
+constexpr size_t decode_mfma_lds_bytes(int head_size) {
+  const size_t tiles = (size_t)kMWaves * 2 * kMTile * head_size * 2;
+  const size_t merge = (size_t)kMWaves * 16 * (2 + head_size) * sizeof(float);  // G <= 16
+  return tiles > merge ? tiles : merge;
+}
+
+// More than 64 KB of dynamic LDS must be granted per kernel (once per device).
+template <auto kKernel>
+hipError_t grant_lds(size_t bytes) {
   static unsigned long long configured = 0;
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (dev >= 64 || !(__atomic_load_n(&configured, __ATOMIC_ACQUIRE) & (1ull << dev))) {
-    e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    e = hipFuncSetAttribute((const void*)kKernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)bytes);
     if (e != hipSuccess) return e;
     if (dev < 64) __atomic_fetch_or(&configured, 1ull << dev, __ATOMIC_RELEASE);
   }
+  return hipSuccess;
+}
+
+template <typename T, int D, bool PAGED>
+hipError_t launch_whole(const DecodeArgs& a, hipStream_t stream) {
+  const long blocks = (long)a.n_rows * a.Hkv;
+  constexpr size_t lds = decode_mfma_lds_bytes(D);
+  hipError_t e = grant_lds<decode_mfma_kernel<T, D, PAGED>>(lds);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL((decode_mfma_kernel<T, D, PAGED>), dim3((unsigned)blocks), dim3(kMThreads),
                      lds, stream, a);
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------- split rows
+// Every launch that is not one whole row per CU: split rows, and rows fewer than the CUs.
+// A workgroup of NW waves owns one (row, kv head, split); wave w takes the 16-token tiles w,
+// w + NW, ... of the split.  Per tile and wave:
+//   S^T[16 x 16] = K . Q^T        D/32 v_mfma_f32_16x16x32
+//   O^T[D x 16] += V^T . P^T      D/16 v_mfma_f32_16x16x16 (bf16: two, P = hi + lo); the S^T
+//                                 accumulator (tokens 4 g + i) is the B layout of P^T
+// V goes through an LDS tile per wave for the transposing reads.  The next tile's K is
+// requested once the current one is used, its V once the current rows are in LDS.
+// Two shapes:
+//  * NW = 8, few workgroups: bound by latency, the chain of round trips (length, K and V,
+//    merge) and a CU's ~36 GB/s.  K pieces go from global memory straight to the MFMA operand
+//    layout (lane (n, g): row n, chunk 4 j + g), and one barrier suffices: the waves' (m, l)
+//    and unscaled O go to LDS together.
+//  * NW = 4, many workgroups: bound by HBM.  K rows are loaded whole (1 KB of consecutive rows
+//    per instruction, nontemporal) and turned in LDS like the whole-row kernel's: with KV
+//    that the last-level cache does not hold, batch 31, 32/8 heads, bf16, lengths U[512, 4096]
+//    61.2 -> 56.5 us against the K pieces' 64-byte segments (59.8); the waves' results then
+//    share the tiles' space (four workgroups fit a CU).
+// Against the dot-product kernel (decode.hip), split + merge, us: one row of 4096, 32/8 heads,
+// fp16 11.5 -> 9.1; 28/4 heads, bf16, batch 5, lengths U[2048, 16000] 45.8 -> 30.5; 12/2 heads,
+// bf16, batch 64, lengths U[300, 4000] 57.9 -> 39.9.
+constexpr int kSTile = 16;
+
+// LDS of a split workgroup: the waves' V (and K) tiles, then (m, l) [NW][16][2] and O [NW][G][D],
+// which share the tiles' space for NW = 4.
+template <int D, int NW>
+constexpr size_t split_lds(int G) {
+  const size_t tiles = (size_t)NW * (NW == 4 ? 2 : 1) * kSTile * D * 2;
+  const size_t merge = (size_t)NW * (16 * 2 + G * D) * sizeof(float);
+  return NW == 4 ? (tiles > merge ? tiles : merge) : tiles + merge;
+}
+
+template <typename T>
+__device__ __forceinline__ f32x4 mfma16k16(const u32x2& a, const u32x2& b, const f32x4& c);
+template <>
+__device__ __forceinline__ f32x4 mfma16k16<f16>(const u32x2& a, const u32x2& b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a),
+                                               __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
+}
+template <>
+__device__ __forceinline__ f32x4 mfma16k16<bf16>(const u32x2& a, const u32x2& b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a),
+                                                   __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+}
+
+template <typename T, int D, bool PAGED, int NW>
+__global__ void __launch_bounds__(NW * kWave, 4) decode_split_mfma_kernel(DecodeArgs a) {
+  constexpr int kThreads = NW * kWave;
+  constexpr int NQK = D / 32;  // QK^T MFMAs (16-byte K pieces per token)
+  constexpr int NDT = D / 16;  // 16-wide output tiles of O^T
+  constexpr bool kKLds = NW == 4;  // K through LDS (above)
+  constexpr bool kBf16 = std::is_same<T, bf16>::value;
+  static_assert(D == 64 || D == 128, "head size 64 or 128");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+
+  int bid = blockIdx.x;
+  const int kvh = bid % a.Hkv;
+  bid /= a.Hkv;
+  const int split = bid % a.max_splits;
+  const int row = bid / a.max_splits;
+  const int G = a.kv_mul;
+  const int h0 = kvh * G;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 15;  // head column / token of the tile / V^T dimension
+  const int g = lane >> 4;  // 16-byte piece group
+
+  // B operand of QK^T MFMA j: lane (n, g) holds q[head h0 + n][32 j + 8 g .. +7] (zero for
+  // columns n >= G).  Requested before the row's length is known.
+  u32x4 qf[NQK];
+  {
+    const T* qp = reinterpret_cast<const T*>(a.q) + (long)row * a.q_row_stride +
+                  (long)(h0 + min(n, G - 1)) * a.q_head_stride + 8 * g;
+#pragma unroll
+    for (int j = 0; j < NQK; ++j) qf[j] = *reinterpret_cast<const u32x4*>(qp + 32 * j);
+  }
+
+  const int len = row_len(a, row);
+  const int st = row_split_tokens(a, len);
+  T* out = reinterpret_cast<T*>(a.o) + (long)row * a.o_row_stride;
+  if (len > a.len_cap || len <= 0) {  // past the launch bound: NaN; empty row: zeros
+    if (split == 0) {
+      const float fill = len > 0 ? __builtin_nanf("") : 0.f;
+      for (int i = threadIdx.x; i < G * D; i += kThreads)
+        out[(long)(h0 + i / D) * a.o_head_stride + i % D] = from_f32<T>(fill);
+    }
+    return;
+  }
+  if ((long)split * st >= len) return;
+  const int s0 = split * st;
+  const int s1 = min(s0 + st, len);
+
+  // ---------------------------------------------------------------- address map
+  const long tok_bytes = a.kv_tok_stride * (long)sizeof(T);
+  const char* kbase = reinterpret_cast<const char*>(a.k) + a.kv_head_stride * (long)sizeof(T) * kvh;
+  const char* vbase = reinterpret_cast<const char*>(a.v) + a.kv_head_stride * (long)sizeof(T) * kvh;
+  const __attribute__((address_space(4))) int* bt = nullptr;
+  long blk_bytes = 0;
+  int bmask = 0;
+  if constexpr (PAGED) {
+    bt = (const __attribute__((address_space(4))) int*)(a.block_table + (long)row * a.bt_row_stride);
+    blk_bytes = a.block_stride * (long)sizeof(T);
+    bmask = (1 << a.bs_log2) - 1;
+  } else {
+    const long base = (long)row * a.kv_row_stride;
+    kbase += base * (long)sizeof(T);
+    vbase += base * (long)sizeof(T);
+  }
+  // Byte offset of token t's row (t in the tile at t0, clamped to the split by the caller); the
+  // two 8-token halves of a tile each lie in one block.
+  struct Blocks { int b[2]; };
+  auto tile_blocks = [&](int t0) __attribute__((always_inline)) {
+    Blocks r;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) r.b[q] = PAGED ? bt[min(t0 + 8 * q, s1 - 1) >> a.bs_log2] : 0;
+    return r;
+  };
+  auto row_off = [&](int t, int t0, const Blocks& bl) __attribute__((always_inline)) {
+    const int tc = min(t, s1 - 1);
+    if constexpr (PAGED)
+      return (long)(tc >= t0 + 8 ? bl.b[1] : bl.b[0]) * blk_bytes + (long)(tc & bmask) * tok_bytes;
+    return (long)tc * tok_bytes;
+  };
+
+  // Per-wave V tile: 16 rows of D elements, chunk c of row r at c ^ (2r & 14); K tile the same
+  // with chunk c at c ^ r (D 64: c ^ (r / 2)).
+  constexpr int CPR = D / 8;        // 16-byte chunks per row
+  constexpr int RPI = kWave / CPR;  // rows per load instruction
+  constexpr int NLV = kSTile / RPI; // whole-row load instructions per tile
+  char* const vt = smem + wave * ((kKLds ? 2 : 1) * kSTile * D * 2);
+  char* const kt = vt + kSTile * D * 2;
+  const int lrow = lane / CPR, lchunk = lane % CPR;
+  auto vt_chunk = [&](int r, int c) __attribute__((always_inline)) {
+    return r * (D * 2) + ((c ^ ((2 * r) & (CPR - 1) & 14)) * 16);
+  };
+  auto kt_chunk = [&](int r, int c) __attribute__((always_inline)) {
+    return r * (D * 2) + ((c ^ ((D == 128 ? r : (r >> 1)) & (CPR - 1))) * 16);
+  };
+  const int tr_e = n >> 2, tr_q = n & 3;
+
+  constexpr int NLK = kKLds ? NLV : NQK;  // (equal)
+  u32x4 kr[NLK], vr[NLV];
+  auto load_k = [&](int t0, const Blocks& bl) __attribute__((always_inline)) {
+    if constexpr (kKLds) {
+#pragma unroll
+      for (int i = 0; i < NLK; ++i)
+        kr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(
+            kbase + row_off(t0 + RPI * i + lrow, t0, bl) + 16 * lchunk));
+    } else {
+      const char* p = kbase + row_off(t0 + n, t0, bl) + 16 * g;
+#pragma unroll
+      for (int j = 0; j < NLK; ++j)
+        kr[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + 64 * j));
+    }
+  };
+  auto load_v = [&](int t0, const Blocks& bl) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NLV; ++i)
+      vr[i] = __builtin_nontemporal_load(
+          reinterpret_cast<const u32x4*>(vbase + row_off(t0 + RPI * i + lrow, t0, bl) + 16 * lchunk));
+  };
+
+  f32x4 oacc[NDT];
+#pragma unroll
+  for (int t = 0; t < NDT; ++t) oacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, lsum = 0.f;
+  const float c = a.scale_log2;
+  typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+  typedef __attribute__((address_space(3))) char lds_char;
+
+  int t0 = s0 + wave * kSTile;
+  if (t0 < s1) {
+    Blocks bl = tile_blocks(t0);
+    load_k(t0, bl);
+    load_v(t0, bl);
+    while (true) {
+      const int tn = t0 + NW * kSTile;
+      const bool more = tn < s1;
+      if (more) bl = tile_blocks(tn);
+      if constexpr (kKLds) {
+#pragma unroll
+        for (int i = 0; i < NLK; ++i)
+          *reinterpret_cast<lds_u32x4*>((lds_char*)(kt + kt_chunk(RPI * i + lrow, lchunk))) = kr[i];
+      }
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NQK; ++j) {
+        u32x4 kf;
+        if constexpr (kKLds)
+          kf = *reinterpret_cast<const lds_u32x4*>((lds_char*)(kt + kt_chunk(n, 4 * j + g)));
+        else
+          kf = kr[j];
+        s = mfma16<T>(kf, qf[j], s);
+      }
+      if (more) load_k(tn, bl);
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = t0 + 4 * g + i < s1 ? s[i] * c : -INFINITY;
+#pragma unroll
+      for (int i = 0; i < NLV; ++i)
+        *reinterpret_cast<lds_u32x4*>((lds_char*)(vt + vt_chunk(RPI * i + lrow, lchunk))) = vr[i];
+      if (more) load_v(tn, bl);
+      bool raise = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) raise |= x[i] - m > kMLazyLog2;
+      if (__builtin_amdgcn_ballot_w64(raise)) {
+        float tm = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+        tm = fmaxf(tm, xor16(tm));
+        tm = fmaxf(tm, partner32(tm));
+        const float mn = fmaxf(m, tm);
+        const float alpha = fast_exp2(m - mn);
+        m = mn;
+        lsum *= alpha;
+#pragma unroll
+        for (int t = 0; t < NDT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) oacc[t][i] *= alpha;
+      }
+      float p[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[i] = fast_exp2(x[i] - m);
+        lsum += p[i];
+      }
+      u32x2 pb, pl;
+      if constexpr (!kBf16) {
+        pb = u32x2{pack2m<f16>(p[0], p[1]), pack2m<f16>(p[2], p[3])};
+      } else {
+        float lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lo[i] = p[i] - (float)(bf16)p[i];
+        pb = u32x2{pack2m<bf16>(p[0], p[1]), pack2m<bf16>(p[2], p[3])};
+        pl = u32x2{pack2m<bf16>(lo[0], lo[1]), pack2m<bf16>(lo[2], lo[3])};
+      }
+#pragma unroll
+      for (int t = 0; t < NDT; ++t) {
+        const int rr = 4 * g + tr_e;
+        const int col = 16 * t + 4 * tr_q;
+        const int off = vt_chunk(rr, col >> 3) + (col & 7) * 2;
+        const s16x4 v4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4*)((__attribute__((address_space(3))) char*)(vt + off)));
+        const u32x2 va = __builtin_bit_cast(u32x2, v4);
+        oacc[t] = mfma16k16<T>(va, pb, oacc[t]);
+        if constexpr (kBf16) oacc[t] = mfma16k16<T>(va, pl, oacc[t]);
+      }
+      if (!more) break;
+      t0 = tn;
+    }
+  }
+
+  // ---------------------------------------------------------------- merge the waves
+  lsum += xor16(lsum);
+  lsum += partner32(lsum);
+  if constexpr (kKLds) __syncthreads();  // every wave is done with its tiles
+  float* s_m = reinterpret_cast<float*>(smem + (kKLds ? 0 : NW * kSTile * D * 2));  // [waves][16]
+  float* s_l = s_m + NW * 16;
+  float* s_o = s_l + NW * 16;  // [waves][G][D]
+  if (g == 0) {
+    s_m[wave * 16 + n] = m;
+    s_l[wave * 16 + n] = lsum;
+  }
+  if (n < G) {
+#pragma unroll
+    for (int t = 0; t < NDT; ++t)
+      *reinterpret_cast<f32x4*>(s_o + (wave * G + n) * D + 16 * t + 4 * g) = oacc[t];
+  }
+  __syncthreads();
+  const bool direct = st >= len;
+  for (int i = threadIdx.x; i < G * D; i += kThreads) {
+    const int hn = i / D, dd = i % D;
+    float mw[NW], M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      mw[w] = s_m[w * 16 + hn];
+      M = fmaxf(M, mw[w]);
+    }
+    float L = 0.f, o = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = fast_exp2(mw[w] - M);
+      L = __builtin_fmaf(f, s_l[w * 16 + hn], L);
+      o = __builtin_fmaf(f, s_o[(w * G + hn) * D + dd], o);
+    }
+    if (direct) {
+      out[(long)(h0 + hn) * a.o_head_stride + dd] = from_f32<T>(o / L);
+    } else {
+      const long pi = ((long)row * a.Hq + h0 + hn) * a.max_splits + split;
+      a.ws[pi * D + dd] = o;
+      if (dd == 0) {
+        float* ml = a.ws + (long)a.n_rows * a.Hq * a.max_splits * D + pi * 2;
+        ml[0] = M;
+        ml[1] = L;
+      }
+    }
+  }
+}
+
+template <typename T, int D, bool PAGED, int NW>
+hipError_t launch_split(const DecodeArgs& a, hipStream_t stream) {
+  const long blocks = (long)a.n_rows * a.Hkv * a.max_splits;
+  const size_t lds = split_lds<D, NW>(a.kv_mul);
+  hipError_t e = grant_lds<decode_split_mfma_kernel<T, D, PAGED, NW>>(split_lds<D, NW>(16));
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((decode_split_mfma_kernel<T, D, PAGED, NW>), dim3((unsigned)blocks),
+                     dim3(NW * kWave), lds, stream, a);
+  return hipGetLastError();
+}
+
+template <typename T, int D, bool PAGED>
+hipError_t launch_p(const DecodeArgs& a, int n_cu, hipStream_t stream) {
+  const long units = (long)a.n_rows * a.Hkv;
+  // Whole rows with a unit per CU or more: the 4-wave kernel that keeps two 32-token tiles of
+  // every wave in flight streams a row fastest.  The single-sequence decode never gets there.
+  if (a.max_splits == 1 && units >= n_cu && a.dyn_splits_log2 < 0)
+    return launch_whole<T, D, PAGED>(a, stream);
+  // Up to two workgroups per CU: the latency shape.  28/4 heads, batch 16, lengths up to 4096,
+  // bf16: 512 workgroups 24.0 us with 8 waves, 23.7 with 4; 1024 workgroups 25.1 and 23.2.
+  return units * a.max_splits <= 2l * n_cu ? launch_split<T, D, PAGED, 8>(a, stream)
+                                           : launch_split<T, D, PAGED, 4>(a, stream);
+}
+
 template <typename T, int D>
-hipError_t launch_t(const DecodeArgs& a, hipStream_t stream) {
-  return a.block_table ? launch_tp<T, D, true>(a, stream) : launch_tp<T, D, false>(a, stream);
+hipError_t launch_t(const DecodeArgs& a, int n_cu, hipStream_t stream) {
+  return a.block_table ? launch_p<T, D, true>(a, n_cu, stream)
+                       : launch_p<T, D, false>(a, n_cu, stream);
 }
 
 }  // namespace
-
-size_t decode_mfma_lds_bytes(int head_size) {
-  const size_t tiles = (size_t)kMWaves * 2 * kMTile * head_size * 2;
-  const size_t merge = (size_t)kMWaves * 16 * (2 + head_size) * sizeof(float);  // G <= 16
-  return tiles > merge ? tiles : merge;
-}
 
 bool decode_mfma_supports(int dtype, int head_size, int kv_mul) {
   return (dtype == kF16 || dtype == kBF16) && (head_size == 64 || head_size == 128) &&
          kv_mul >= 1 && kv_mul <= 16;
 }
 
-hipError_t launch_decode_mfma(const DecodeArgs& a, int dtype, hipStream_t stream) {
+hipError_t launch_decode_mfma(const DecodeArgs& a, int n_cu, int dtype, hipStream_t stream) {
   if (dtype == kF16)
-    return a.head_size == 64 ? launch_t<f16, 64>(a, stream) : launch_t<f16, 128>(a, stream);
-  return a.head_size == 64 ? launch_t<bf16, 64>(a, stream) : launch_t<bf16, 128>(a, stream);
+    return a.head_size == 64 ? launch_t<f16, 64>(a, n_cu, stream)
+                             : launch_t<f16, 128>(a, n_cu, stream);
+  return a.head_size == 64 ? launch_t<bf16, 64>(a, n_cu, stream)
+                           : launch_t<bf16, 128>(a, n_cu, stream);
 }
 
 }  // namespace orin

@@ -28,24 +28,24 @@ struct DecodeArgs {
   int n_seg;
   void* o;  // o(r, h, j) = o[r*o_row_stride + h*o_head_stride + j]
   long o_row_stride, o_head_stride;
-  float* ws;  // [n_rows, Hq, max_splits, head_size + 2] fp32 partials (unused if max_splits == 1)
+  // fp32 partials (unused if max_splits == 1): acc rows [n_rows, Hq, max_splits][head_size], then
+  // (m, l) pairs [n_rows, Hq, max_splits][2]
+  float* ws;
   int max_splits, split_tokens;
+  int dyn_splits_log2;  // >= 0: a row's split size follows its length (row_split_tokens)
   int wide;  // dot-product kernel: 16-wave workgroups where the shape fits (decode.hip)
-  int mfma;  // one split per row and a unit per CU or more: the matrix-core kernel where it
-             // supports the shape (decode_mfma.hip)
   int n_rows, Hq, Hkv, kv_mul, head_size;
   float scale_log2;  // softmax scale * log2(e)
 };
 
 int decode_heads_per_block(int kv_mul);
 bool decode_supports(int dtype, int head_size);
-hipError_t launch_decode(const DecodeArgs& a, int dtype, hipStream_t stream);
+hipError_t launch_decode(const DecodeArgs& a, int n_cu, int dtype, hipStream_t stream);
 // Matrix-core decode (decode_mfma.hip) for 16-bit caches, head sizes 64 / 128 and up to 16
 // query heads per kv head: one workgroup per (row, kv head, split) serving all kv_mul heads.
-// launch_decode routes the shapes it supports there.
+// launch_decode routes every launch it supports there.
 bool decode_mfma_supports(int dtype, int head_size, int kv_mul);
-size_t decode_mfma_lds_bytes(int head_size);
-hipError_t launch_decode_mfma(const DecodeArgs& a, int dtype, hipStream_t stream);
+hipError_t launch_decode_mfma(const DecodeArgs& a, int n_cu, int dtype, hipStream_t stream);
 
 // Tile-parallel attention forward on MFMA (fp16 / bf16): causal prefill over a
 // kuiper-layout cache, or bidirectional varlen segments.
