@@ -98,9 +98,10 @@ int orin_batched_mha(int32_t start_pos, int32_t seq_len, int32_t head_num, int32
  * (kuiper/source/op/kernels/cuda/flash_attention_kernel.cuh:27-80, 143-181).
  * Causal GQA prefill: query/output [seq_len, dim], caches [layers, max_seq_len, kv_dim];
  * row i attends 0..start_pos+i (flash_attention_kernel.cu:575-578).  dtype selects the
- * reference's fp32 or fp16 variant; bf16 is new.  fp16/bf16 run on MFMA.  A 16-bit launch
- * with fewer 256-query blocks than the device has CUs splits the keys of each block and
- * keeps the partials in the stream's library-owned workspace (see below).
+ * reference's fp32 or fp16 variant; bf16 is new.  All run on MFMA.  A larger 16-bit launch
+ * with fewer 256-query blocks than the device has CUs splits the keys of each block over
+ * workgroups and keeps the partials in the stream's library-owned workspace (see below);
+ * small and mid-sized launches need none.
  * bf16 range: the softmax weights and the weighted sum with V run in fp16 (V is converted
  * to fp16 on chip), so bf16 V must satisfy |v| <= 65504; a larger value turns non-finite
  * the outputs of every row that attends to it (and possibly of other rows whose 64-key
@@ -198,8 +199,8 @@ size_t orin_flash_attention_decode_noalloc_max_bytes(void);
  *    other work that uses that stream's buffer runs.
  *
  * orin_flash_attention_decode_workspace_size: decode bytes for a cache of max_seq_len rows
- * (any kv_head_num).  orin_flash_attention_prefill_workspace_size: key-split bytes of one
- * causal prefill launch (0 when it does not split).  orin_attn_workspace_reserve_stream
+ * (any kv_head_num).  orin_flash_attention_prefill_workspace_size: key-split bytes that one
+ * causal prefill launch may need (0: never).  orin_attn_workspace_reserve_stream
  * allocates both on the current device for `stream` now.  orin_attn_workspace_reserve
  * reserves decode bytes for the NULL stream and makes every decode buffer created later on
  * this device at least that large.  orin_attn_workspace_reserve_stream also prepares the

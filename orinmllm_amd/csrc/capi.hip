@@ -509,6 +509,7 @@ static int prefill_common(int32_t start_pos, int32_t seq_len, int32_t head_num,
   a.kv_mul = kv_mul;
   a.head_size = head_size;
   a.scale_log2 = resolve_scale(0.f, head_size) * kLog2e;
+  a.n_cu = device_cus();
   if (fused) {
     // The fused Q producer runs in the ping-pong kernel's Q load (head sizes 64 and 128);
     // it reads the raw query while other rows' outputs are written, so no aliasing.
@@ -520,9 +521,12 @@ static int prefill_common(int32_t start_pos, int32_t seq_len, int32_t head_num,
     a.rope_cos = rope_cos;
     a.eps = eps;
   }
-  // Too few query blocks to fill the device: split their keys (library workspace).
+  // Too few query blocks to fill the device and too much work for the kernel that splits keys
+  // inside the workgroup: split the blocks' keys over workgroups (library workspace).
   size_t split_bytes = 0;
-  const int chunk = fwd_pp_key_split(a, dtype, device_cus(), &split_bytes);
+  const int chunk = fwd_sk_prefers(a, dtype, true)
+                        ? 0
+                        : fwd_pp_key_split(a, dtype, device_cus(), &split_bytes);
   if (chunk > 0) {
     void* ws = nullptr;
     const int st = library_workspace(kWsPrefillSplit, (hipStream_t)stream, split_bytes, &ws);

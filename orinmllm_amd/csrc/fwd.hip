@@ -462,9 +462,10 @@ hipError_t launch_fwd_d(const FwdArgs& a, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
-// Head sizes 64-128 go to the ping-pong kernel (256-query workgroups, one per CU) when its
-// grid covers every CU at least once, or when the caller planned a key split for a causal
-// launch that does not (fwd_pp_key_split).
+// Small and mid-sized launches go to the kernel that splits keys inside the workgroup
+// (fwd_sk_prefers).  The rest of head sizes 64-128 go to the ping-pong kernel (256-query
+// workgroups, one per CU) when its grid covers every CU at least once, or when the caller planned
+// a key split for a causal launch that does not (fwd_pp_key_split).
 template <bool CAUSAL>
 bool use_pp(const FwdArgs& a, int dtype) {
   if (!fwd_pp_supports(a, dtype)) return false;
@@ -476,6 +477,8 @@ bool use_pp(const FwdArgs& a, int dtype) {
 
 template <bool CAUSAL>
 hipError_t launch_fwd(const FwdArgs& a, int dtype, hipStream_t stream) {
+  if (a.key_chunk_tiles == 0 && fwd_sk_prefers(a, dtype, CAUSAL))
+    return launch_fwd_sk(a, dtype, CAUSAL, stream);
   if (use_pp<CAUSAL>(a, dtype)) return launch_fwd_pp(a, dtype, CAUSAL, stream);
   if (dtype == kF16) return launch_fwd_d<CAUSAL, f16>(a, stream);
   if (dtype == kBF16) return launch_fwd_d<CAUSAL, bf16>(a, stream);

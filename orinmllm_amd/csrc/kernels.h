@@ -60,7 +60,7 @@ struct FwdArgs {
   int n_q;        // query rows (causal: seq_len; varlen: total tokens)
   int start_pos;  // causal: query i sits at position start_pos + i
   int causal;     // fp32 kernel (fwd_f32.hip): row i sees keys 0 .. start_pos + i
-  int n_cu;       // fp32 kernel: the device's CUs
+  int n_cu;       // the device's CUs
   const int* cu_seqlens;  // varlen (device), n_seg + 1 entries; null = one segment of n_q
   int n_seg, max_seqlen;
   int Hq, Hkv, kv_mul, head_size;
@@ -90,6 +90,11 @@ hipError_t launch_fwd_varlen(const FwdArgs& a, int dtype, hipStream_t stream);
 // or one bidirectional segment, where it is the faster kernel.
 bool fwd_f32_supports(const FwdArgs& a);
 hipError_t launch_fwd_f32(const FwdArgs& a, hipStream_t stream);
+
+// Keys split inside the workgroup, for small and mid-sized launches (fwd_sk.hip); the launches
+// that run there.  Needs a.n_cu.
+bool fwd_sk_prefers(const FwdArgs& a, int dtype, bool causal);
+hipError_t launch_fwd_sk(const FwdArgs& a, int dtype, bool causal, hipStream_t stream);
 
 // 8-wave ping-pong variant for head sizes 64, 72, 80, 96 and 128 (fwd_pp.hip).
 bool fwd_pp_supports(const FwdArgs& a, int dtype);
