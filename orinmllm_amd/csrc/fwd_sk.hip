@@ -10,12 +10,13 @@
 // most CUs idle.  Here a workgroup of 4 waves owns 32 rows and wave w takes the 32-key tiles w,
 // w + 4, ... with its own online softmax; the waves are merged once through LDS.  The chain is a
 // quarter as long and the blocks are an eighth as large, so the grid fills the chip without a
-// second launch that merges partials.  Rows of the query heads that share a kv head are packed
+// second launch that merges partials.  Where the grid is large enough, a workgroup owns two such
+// sets of 32 rows: each K and V fragment read from LDS serves two products.  Rows of the query heads that share a kv head are packed
 // (row R of a kv head = query R / kv_mul, head R % kv_mul of its group): short prompts fill the
 // 32 rows, and little of a causal diagonal tile is masked.
 //
-// The price: K and V are read from L2 once per 32 rows (a CU streams ~110 GB/s from L2), with no
-// wave sharing another's tile, so large launches stay on fwd_pp.hip.
+// The price: K and V are read from L2 once per 32 or 64 rows (a CU streams ~110 GB/s from L2), with
+// no wave sharing another's tile, so large launches stay on fwd_pp.hip.
 //
 // Per 32-key tile and wave, lane (lq, hf) = (lane % 32, lane / 32):
 //   S^T[key][row] = K . Q^T      D/16 v_mfma_f32_32x32x16; lane: row lq, 16 keys
@@ -28,6 +29,7 @@
 // fp16 after the LDS read (the softmax weights are fp16, see common.h).
 // Head sizes below 128 pad the QK contraction to a multiple of 16 (zero Q elements) and O^T to a
 // multiple of 32 (rows never stored).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -38,7 +40,6 @@ namespace orin {
 
 namespace {
 
-constexpr int kSkRows = 32;                   // rows per workgroup
 constexpr int kSkKeys = 32;                   // keys per wave tile
 
 // LDS rows of a K or V tile, in 16-byte chunks.  Head size 128: 16, chunk c of row r at c ^ (r & 15)
@@ -50,26 +51,30 @@ template <int D>
 constexpr int sk_row_chunks() { return D == 128 ? 16 : D == 96 ? 13 : D == 64 ? 9 : 10; }
 template <int D>
 constexpr int sk_transfers() { return (kSkKeys * sk_row_chunks<D>() + kWave - 1) / kWave; }
-// K and V tiles of the waves (1 KB per transfer), or O [wave][row][DT * 32] in the merge; then the
-// waves' (m, l).
+// K and V tiles of the waves (1 KB per transfer), or O [wave][32 rows][DT * 32] in the merge; then
+// the Q fragments of two row sets, or the waves' (m, l).
 template <int D, int NW>
-constexpr int sk_ml_offset() {
+constexpr int sk_q_offset() {
   const int tiles = NW * 2 * sk_transfers<D>() * 1024;
-  const int merge = NW * kSkRows * ((D + 31) / 32 * 32) * 4;
+  const int merge = NW * 32 * ((D + 31) / 32 * 32) * 4;
   return tiles > merge ? tiles : merge;
 }
-template <int D, int NW>
-constexpr int sk_lds() { return sk_ml_offset<D, NW>() + NW * kSkRows * 2 * 4; }
+template <int D, int RS, int NW>
+constexpr int sk_lds() {
+  const int q = RS > 1 ? RS * ((D + 15) / 16) * 1024 : 0, ml = NW * 32 * RS * 2 * 4;
+  return sk_q_offset<D, NW>() + (q > ml ? q : ml);
+}
 // A lane's 16 weights of one tile may sum to at most this before the row maximum is raised.
 constexpr float kSkSumMax = 256.0f;
 
 // FQ: the query rows are raw and the Q producer runs on the fragments (a.rope_sin set).
-template <typename T, bool CAUSAL, int D, bool FQ, int NW>
+template <typename T, bool CAUSAL, int D, bool FQ, int RS, int NW>
 __global__ void __launch_bounds__(NW * kWave, 2) fwd_sk_kernel(FwdArgs a) {
   constexpr int QS = (D + 15) / 16;  // 16-wide slices of the QK contraction
   constexpr int DT = (D + 31) / 32;  // 32-wide output tiles of O^T
   constexpr int NCH = D / 8;         // valid 16-byte chunks of a K / V row
   constexpr bool kConvV = !std::is_same<T, f16>::value;
+  constexpr int kSkRows = 32 * RS;   // rows per workgroup
   constexpr int RC = sk_row_chunks<D>(), NI = sk_transfers<D>();
   constexpr int kTile = NI * 1024;  // bytes of a K or V tile
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -105,11 +110,15 @@ __global__ void __launch_bounds__(NW * kWave, 2) fwd_sk_kernel(FwdArgs a) {
   const int r_last = min(r_first + kSkRows, rows) - 1;
   kv_len = CAUSAL ? a.start_pos + r_last / G + 1 : rows / G;
   const int n_tiles = (kv_len + kSkKeys - 1) / kSkKeys;
-  // This lane's row (rows past the end repeat the last one and are not stored).
-  const int R = min(r_first + lq, r_last);
-  const int tok = R / G;
-  const int head = kvh * G + R % G;
-  const int pos = CAUSAL ? a.start_pos + tok : kv_len - 1;          // last key of the row
+  // This lane's row of each set (rows past the end repeat the last one and are not stored).
+  int tok[RS], head[RS], pos[RS];  // pos: the last key the row sees
+#pragma unroll
+  for (int u = 0; u < RS; ++u) {
+    const int R = min(r_first + 32 * u + lq, r_last);
+    tok[u] = R / G;
+    head[u] = kvh * G + R % G;
+    pos[u] = CAUSAL ? a.start_pos + tok[u] : kv_len - 1;
+  }
   const int pos_min = CAUSAL ? a.start_pos + r_first / G : kv_len - 1;
 
   const long tstr = a.kv_tok_stride;
@@ -141,24 +150,18 @@ __global__ void __launch_bounds__(NW * kWave, 2) fwd_sk_kernel(FwdArgs a) {
     k_off[b] = __umul24(D == 128 ? lane >> 4 : chunk_row(b), row_bytes) + chunk_col(b, false);
   const uint32_t v_off = D == 128 ? __umul24(lane >> 4, row_bytes) + chunk_col(0, true) : 0u;
   char* const my = smem + wave * 2 * kTile;
-  const lds_ptr k_lds = (lds_ptr)my, v_lds = k_lds + kTile;
   const uint32_t k_addr = __builtin_amdgcn_readfirstlane(lds_addr(my));
   auto issue = [&](const T* x, int t0, auto is_v) __attribute__((always_inline)) {
     constexpr bool V = decltype(is_v)::value;
     const uint32_t dst = k_addr + (V ? kTile : 0);
     const char* base = reinterpret_cast<const char*>(x + (long)t0 * tstr);
-    if (t0 + kSkKeys <= kv_len) {
+    // Rows past the sequence read the last chunk of its last row: finite values, in bounds.
+    const uint32_t lim =
+        (uint32_t)min(kv_len - 1 - t0, kSkKeys - 1) * row_bytes + (D - 8) * (uint32_t)sizeof(T);
 #pragma unroll
-      for (int b = 0; b < NI; ++b) {
-        const uint32_t off =
-            D == 128 ? (V ? v_off : k_off[b & 3]) + 4 * b * row_bytes : k_off[b % NOK];
-        dma16_s(base, off, dst + b * 1024);
-      }
-    } else {  // the last tile: rows past the sequence read its last row
-#pragma unroll
-      for (int b = 0; b < NI; ++b)
-        dma16_s(base, __umul24(min(chunk_row(b), kv_len - 1 - t0), row_bytes) + chunk_col(b, V),
-                dst + b * 1024);
+    for (int b = 0; b < NI; ++b) {
+      const uint32_t off = D == 128 ? (V ? v_off : k_off[b & 3]) + 4 * b * row_bytes : k_off[b % NOK];
+      dma16_s(base, min(off, lim), dst + b * 1024);
     }
   };
   auto issue_k = [&](int t0) __attribute__((always_inline)) { issue(kb, t0, std::false_type{}); };
@@ -169,44 +172,70 @@ __global__ void __launch_bounds__(NW * kWave, 2) fwd_sk_kernel(FwdArgs a) {
   if (any) issue_k(t * kSkKeys);
 
   // ------------------------------------------------------------ Q fragments
+  // One row set: in registers.  Two: wave u loads set u and all waves read the fragments from
+  // LDS ([set][slice][lane]), which leaves the registers to O.
   u32x4 qf[QS];
-  {
-    const T* qp = reinterpret_cast<const T*>(a.q) + (long)(seg_start + tok) * a.q_tok_stride +
-                  (long)head * a.q_head_stride;
+  char* const q_sm = smem + sk_q_offset<D, NW>();
+#pragma unroll
+  for (int u = 0; u < RS; ++u) {
+    if (RS > 1 && wave != u) continue;
+    const T* qp = reinterpret_cast<const T*>(a.q) + (long)(seg_start + tok[u]) * a.q_tok_stride +
+                  (long)head[u] * a.q_head_stride;
 #pragma unroll
     for (int s = 0; s < QS; ++s) {
       u32x4 val = {0u, 0u, 0u, 0u};
       if (16 * s + 8 * hf < D) val = *reinterpret_cast<const u32x4*>(qp + 16 * s + 8 * hf);
       qf[s] = val;
     }
-  }
-  if constexpr (FQ && CAUSAL && (D == 64 || D == 128))
-    fuse_q_producer<T, D>(a, qf, true, pos, pos, hf);
+    if constexpr (FQ && CAUSAL && (D == 64 || D == 128))
+      fuse_q_producer<T, D>(a, qf, true, pos[u], pos[u], hf);
 #pragma unroll
-  for (int s = 0; s < QS; ++s) __asm__ volatile("" : "+v"(qf[s]));  // Q has arrived
+    for (int s = 0; s < QS; ++s) __asm__ volatile("" : "+v"(qf[s]));  // Q has arrived
+    if constexpr (RS > 1) {
+#pragma unroll
+      for (int s = 0; s < QS; ++s)
+        *reinterpret_cast<u32x4*>(q_sm + ((u * QS + s) * 64 + lane) * 16) = qf[s];
+    }
+  }
+  if constexpr (RS > 1) __syncthreads();
+  const lds_ptr q_p = (lds_ptr)(q_sm + lane * 16);
+  auto q_frag = [&](int u, int s) __attribute__((always_inline)) {
+    if constexpr (RS > 1) return lds_read128(q_p, (u * QS + s) * 1024);
+    return qf[s];
+  };
   if (any) issue_v(t * kSkKeys);
 
   // Fragment addresses.  K fragment s: row lq, chunk 2s + hf.  V^T fragment (chunk ck of 16
   // keys, tile dt): lane L = 16g + 4e + q reads row 16 ck + 4(g/2) + e (+8 for the second half)
   // and columns dt*32 + 16(g&1) + 4q .. +3.
-  lds_ptr k_p[QS], v_p[DT];
-#pragma unroll
-  for (int s = 0; s < QS; ++s)
-    k_p[s] = k_lds + lq * RC * 16 + (D == 128 ? (2 * s + hf) ^ (lq & 15) : 2 * s + hf) * 16;
+  // At head size 128 (256-byte rows, tiles at multiples of 1 KB) the swizzle makes fragment s
+  // (tile dt) the first one's address with 32 s (64 dt) flipped.
+  const lds_ptr k_lds = (lds_ptr)my, v_lds = k_lds + kTile;
+  uint32_t k_a = lq * RC * 16 + (D == 128 ? hf ^ (lq & 15) : hf) * 16;
+  uint32_t v_a;
   {
     const int g = lane >> 4, e = (lane >> 2) & 3, q = lane & 3;
-    const int row = 4 * (g >> 1) + e;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-      v_p[dt] = v_lds + row * RC * 16 + (D == 128 ? dt ^ e : dt) * 64 + (g & 1) * 32 + q * 8;
+    v_a = (4 * (g >> 1) + e) * RC * 16 + (D == 128 ? e : 0) * 64 + (g & 1) * 32 + q * 8;
   }
+  auto k_p = [&](int s) __attribute__((always_inline)) {
+    return k_lds + (D == 128 ? k_a ^ (32 * s) : k_a + 32 * s);
+  };
+  auto v_p = [&](int dt) __attribute__((always_inline)) {
+    return v_lds + (D == 128 ? v_a ^ (64 * dt) : v_a + 64 * dt);
+  };
 
-  f32x16 oacc[DT];
+  constexpr int kVAhead = DT < 2 ? 2 : 3;  // V fragments read ahead of their products
+  f32x16 oacc[RS][DT];
+  // Running row maximum times the scale (log2 units) and this half's weights.
+  float mc[RS], l[RS];
 #pragma unroll
-  for (int d = 0; d < DT; ++d)
+  for (int u = 0; u < RS; ++u) {
+    mc[u] = l[u] = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) oacc[d][r] = 0.f;
-  float mc = 0.f, l = 0.f;  // running row maximum times the scale (log2 units), this half's weights
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[u][d][r] = 0.f;
+  }
   const float c = a.scale_log2;
   bool first = true;
 
@@ -214,78 +243,100 @@ __global__ void __launch_bounds__(NW * kWave, 2) fwd_sk_kernel(FwdArgs a) {
     for (;;) {
       const int t0 = t * kSkKeys;
       const bool more = t + NW < n_tiles;
+      // Two row sets and V's conversion: the fragment addresses are formed where they are used,
+      // not kept in registers (24 spilled otherwise).
+      if constexpr (RS > 1 && kConvV) __asm__ volatile("" : "+v"(k_a), "+v"(v_a));
       // ---- S^T (K landed; the younger V transfers may be in flight)
       __builtin_amdgcn_sched_barrier(0);
       wait_vmcnt<NI>();
       __builtin_amdgcn_sched_barrier(0);
-      f32x16 s;
+      f32x16 s[RS];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = 0.f;
+      for (int u = 0; u < RS; ++u)
 #pragma unroll
-      for (int i = 0; i < QS; ++i) s = mfma32<T>(lds_read128(k_p[i], 0), qf[i], s);
+        for (int r = 0; r < 16; ++r) s[u][r] = 0.f;
+#pragma unroll
+      for (int i = 0; i < QS; ++i) {
+        const u32x4 kf = lds_read128(k_p(i), 0);
+#pragma unroll
+        for (int u = 0; u < RS; ++u) s[u] = mfma32<T>(kf, q_frag(u, i), s[u]);
+      }
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the K tile has been read
       if (more) issue_k(t0 + NW * kSkKeys);
 
       // ---- softmax: P = 2^(c s - mc) with the running maximum left as it is while no weight
       // sum of a lane passes 2^8; else, and on the first tile, the row maximum is taken.
-      if (t0 + kSkKeys - 1 > pos_min) {
-        const int rel = pos - t0 - 4 * hf;
+      u32x4 pf[RS][2];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int cr = 8 * (r >> 2) + (r & 3);
-          s[r] = cr > rel ? -INFINITY : s[r];
+      for (int u = 0; u < RS; ++u) {
+        if (t0 + kSkKeys - 1 > pos_min) {
+          const int rel = pos[u] - t0 - 4 * hf;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int cr = 8 * (r >> 2) + (r & 3);
+            s[u][r] = cr > rel ? -INFINITY : s[u][r];
+          }
         }
-      }
-      u32x4 pf[2];
-      float ls;
-      auto weights = [&]() __attribute__((always_inline)) {
-        float lsp[4] = {0.f, 0.f, 0.f, 0.f};
+        float ls;
+        auto weights = [&]() __attribute__((always_inline)) {
+          float lsp[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          const uint32_t pk = pack2<f16>(fast_exp2(__builtin_fmaf(s[r], c, -mc)),
-                                         fast_exp2(__builtin_fmaf(s[r + 1], c, -mc)));
-          pf[r >> 3][(r & 7) >> 1] = pk;
-          lsp[(r >> 1) & 3] = sum_pair<f16>(pk, lsp[(r >> 1) & 3]);
+          for (int r = 0; r < 16; r += 2) {
+            const uint32_t pk = pack2<f16>(fast_exp2(__builtin_fmaf(s[u][r], c, -mc[u])),
+                                           fast_exp2(__builtin_fmaf(s[u][r + 1], c, -mc[u])));
+            pf[u][r >> 3][(r & 7) >> 1] = pk;
+            lsp[(r >> 1) & 3] = sum_pair<f16>(pk, lsp[(r >> 1) & 3]);
+          }
+          ls = (lsp[0] + lsp[1]) + (lsp[2] + lsp[3]);
+        };
+        if (!first) weights();
+        if (first || __builtin_amdgcn_ballot_w64(!(ls <= kSkSumMax))) {
+          float mx = s[u][0];
+#pragma unroll
+          for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[u][r]);
+          mx = fmaxf(mx, partner32(mx)) * c;
+          if (first) {
+            mc[u] = mx > -INFINITY ? mx : 0.f;  // no visible key yet: none later either
+          } else {
+            const float mn = fmaxf(mc[u], mx);
+            const float alpha = fast_exp2(mc[u] - mn);
+            mc[u] = mn;
+            l[u] *= alpha;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+              for (int r = 0; r < 16; ++r) oacc[u][d][r] *= alpha;
+          }
+          weights();
         }
-        ls = (lsp[0] + lsp[1]) + (lsp[2] + lsp[3]);
-      };
-      if (!first) weights();
-      if (first || __builtin_amdgcn_ballot_w64(!(ls <= kSkSumMax))) {
-        float mx = s[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-        mx = fmaxf(mx, partner32(mx)) * c;
-        if (first) {
-          mc = mx > -INFINITY ? mx : 0.f;  // no visible key yet: none later either
-        } else {
-          const float mn = fmaxf(mc, mx);
-          const float alpha = fast_exp2(mc - mn);
-          mc = mn;
-          l *= alpha;
-#pragma unroll
-          for (int d = 0; d < DT; ++d)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) oacc[d][r] *= alpha;
-        }
-        weights();
+        l[u] += ls;
       }
       first = false;
-      l += ls;
 
       // ---- O^T (V landed; the younger K transfers may be in flight)
       if (more) wait_vmcnt<NI>();
       else wait_vmcnt<0>();
       __builtin_amdgcn_sched_barrier(0);
+      auto v_frag = [&](int i) __attribute__((always_inline)) {
+        const int dt = i % DT, row = i / DT * 16;
+        const u32x2 lo = lds_read_tr(v_p(dt), row * RC * 16);
+        const u32x2 hi = lds_read_tr(v_p(dt), (row + 8) * RC * 16);
+        return u32x4{lo[0], lo[1], hi[0], hi[1]};
+      };
+      u32x4 vr[kVAhead];
 #pragma unroll
-      for (int ck = 0; ck < 2; ++ck)
+      for (int i = 0; i < kVAhead; ++i) vr[i] = v_frag(i);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const u32x2 lo = lds_read_tr(v_p[dt], ck * 16 * RC * 16);
-          const u32x2 hi = lds_read_tr(v_p[dt], (ck * 16 + 8) * RC * 16);
-          u32x4 vf = {lo[0], lo[1], hi[0], hi[1]};
-          if constexpr (kConvV) vf = bf16x8_to_f16x8(vf);
-          oacc[dt] = mfma32<f16>(vf, pf[ck], oacc[dt]);
-        }
+      for (int i = 0; i < 2 * DT; ++i) {
+        u32x4 vf = vr[i % kVAhead];
+        if constexpr (kConvV) vf = bf16x8_to_f16x8(vf);
+        if (i + kVAhead < 2 * DT) vr[i % kVAhead] = v_frag(i + kVAhead);
+#pragma unroll
+        for (int u = 0; u < RS; ++u)
+          oacc[u][i % DT] = mfma32<f16>(vf, pf[u][i / DT], oacc[u][i % DT]);
+        // Two row sets leave no registers for the scheduler to gather the conversions early.
+        if constexpr (RS > 1 && kConvV) __builtin_amdgcn_sched_barrier(0);
+      }
       if (!more) break;
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the V tile has been read
       t += NW;
@@ -293,72 +344,77 @@ __global__ void __launch_bounds__(NW * kWave, 2) fwd_sk_kernel(FwdArgs a) {
     }
 
   // ------------------------------------------------------------ merge the waves and store
-  // O [wave][row][DT * 32], 4-float chunk ch of a row at ch ^ row within its group of 8.
-  const float l_row = l + partner32(l);
-  const float m_row = l_row > 0.f ? mc : -INFINITY;  // a wave whose keys are all masked
-  __syncthreads();  // every wave is done with its tiles
+  // O [wave][row][DT * 32] of one row set at a time, 4-float chunk ch of a row at ch ^ row within
+  // its group of 8; (m, l) [wave][kSkRows][2] take the Q fragments' place.
   constexpr int OW = DT * 32;
   float* s_o = reinterpret_cast<float*>(smem);
-  float* s_ml = reinterpret_cast<float*>(smem + sk_ml_offset<D, NW>());
-  if (hf == 0) {
-    s_ml[(wave * kSkRows + lq) * 2] = m_row;
-    s_ml[(wave * kSkRows + lq) * 2 + 1] = l_row;
-  }
+  float* s_ml = reinterpret_cast<float*>(q_sm);
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-      const int ch = dt * 8 + ((2 * rg + hf) ^ (lq & 7));
-      *reinterpret_cast<f32x4*>(s_o + (wave * kSkRows + lq) * OW + ch * 4) =
-          f32x4{oacc[dt][4 * rg], oacc[dt][4 * rg + 1], oacc[dt][4 * rg + 2], oacc[dt][4 * rg + 3]};
+  for (int u = 0; u < RS; ++u) {
+    const float l_row = l[u] + partner32(l[u]);
+    const float m_row = l_row > 0.f ? mc[u] : -INFINITY;  // a wave whose keys are all masked
+    __syncthreads();  // every wave is done with its tiles (u > 0: with the last set's O)
+    if (hf == 0) {
+      s_ml[(wave * kSkRows + 32 * u + lq) * 2] = m_row;
+      s_ml[(wave * kSkRows + 32 * u + lq) * 2 + 1] = l_row;
     }
-  __syncthreads();
-  for (int x = threadIdx.x; x < kSkRows * NCH; x += NW * kWave) {
-    const int row = x / NCH, c8 = x % NCH;  // 8 dimensions of a row
-    const int Ro = r_first + row;
-    if (Ro > r_last) break;
-    float M = -INFINITY, mw[NW];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      mw[w] = s_ml[(w * kSkRows + row) * 2];
-      M = fmaxf(M, mw[w]);
-    }
-    const float Mu = M > -INFINITY ? M : 0.f;
-    float L = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float f = fast_exp2(mw[w] - Mu);
-      L = __builtin_fmaf(f, s_ml[(w * kSkRows + row) * 2 + 1], L);
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int lc = 2 * c8 + q, ch = (lc & ~7) + ((lc & 7) ^ (row & 7));
-        const f32x4 y = *reinterpret_cast<const f32x4*>(s_o + (w * kSkRows + row) * OW + ch * 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[4 * q + e] = __builtin_fmaf(f, y[e], o[4 * q + e]);
+      for (int rg = 0; rg < 4; ++rg) {
+        const int ch = dt * 8 + ((2 * rg + hf) ^ (lq & 7));
+        *reinterpret_cast<f32x4*>(s_o + (wave * 32 + lq) * OW + ch * 4) =
+            f32x4{oacc[u][dt][4 * rg], oacc[u][dt][4 * rg + 1], oacc[u][dt][4 * rg + 2],
+                  oacc[u][dt][4 * rg + 3]};
       }
+    __syncthreads();
+    for (int x = threadIdx.x; x < 32 * NCH; x += NW * kWave) {
+      const int row = x / NCH, c8 = x % NCH;  // 8 dimensions of a row
+      const int Ro = r_first + 32 * u + row;
+      if (Ro > r_last) break;
+      float M = -INFINITY, mw[NW];
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        mw[w] = s_ml[(w * kSkRows + 32 * u + row) * 2];
+        M = fmaxf(M, mw[w]);
+      }
+      const float Mu = M > -INFINITY ? M : 0.f;
+      float L = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float f = fast_exp2(mw[w] - Mu);
+        L = __builtin_fmaf(f, s_ml[(w * kSkRows + 32 * u + row) * 2 + 1], L);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int lc = 2 * c8 + q, ch = (lc & ~7) + ((lc & 7) ^ (row & 7));
+          const f32x4 y = *reinterpret_cast<const f32x4*>(s_o + (w * 32 + row) * OW + ch * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[4 * q + e] = __builtin_fmaf(f, y[e], o[4 * q + e]);
+        }
+      }
+      const float inv = 1.f / L;
+      const int to = Ro / G;
+      T* op = reinterpret_cast<T*>(a.o) + (long)(seg_start + to) * a.o_tok_stride +
+              (long)(kvh * G + Ro % G) * a.o_head_stride + 8 * c8;
+      *reinterpret_cast<u32x4*>(op) =
+          u32x4{pack2<T>(o[0] * inv, o[1] * inv), pack2<T>(o[2] * inv, o[3] * inv),
+                pack2<T>(o[4] * inv, o[5] * inv), pack2<T>(o[6] * inv, o[7] * inv)};
     }
-    const float inv = 1.f / L;
-    const int to = Ro / G;
-    T* op = reinterpret_cast<T*>(a.o) + (long)(seg_start + to) * a.o_tok_stride +
-            (long)(kvh * G + Ro % G) * a.o_head_stride + 8 * c8;
-    *reinterpret_cast<u32x4*>(op) =
-        u32x4{pack2<T>(o[0] * inv, o[1] * inv), pack2<T>(o[2] * inv, o[3] * inv),
-              pack2<T>(o[4] * inv, o[5] * inv), pack2<T>(o[6] * inv, o[7] * inv)};
   }
 }
 
 template <bool CAUSAL>
-long sk_blocks(const FwdArgs& a) {
-  const long tiles = ((long)(CAUSAL ? a.n_q : a.max_seqlen) * a.kv_mul + kSkRows - 1) / kSkRows;
+long sk_blocks(const FwdArgs& a, int rows) {
+  const long tiles = ((long)(CAUSAL ? a.n_q : a.max_seqlen) * a.kv_mul + rows - 1) / rows;
   return tiles * a.Hkv * (CAUSAL ? 1 : a.n_seg);
 }
 
-template <typename T, bool CAUSAL, int D, bool FQ, int NW>
+template <typename T, bool CAUSAL, int D, bool FQ, int RS, int NW>
 hipError_t launch_sk_t(const FwdArgs& a, hipStream_t stream) {
-  const long blocks = sk_blocks<CAUSAL>(a);
+  const long blocks = sk_blocks<CAUSAL>(a, 32 * RS);
   if (blocks <= 0) return hipSuccess;
-  constexpr int lds = sk_lds<D, NW>();
-  const void* fn = (const void*)fwd_sk_kernel<T, CAUSAL, D, FQ, NW>;
+  constexpr int lds = sk_lds<D, RS, NW>();
+  const void* fn = (const void*)fwd_sk_kernel<T, CAUSAL, D, FQ, RS, NW>;
   // More than 64 KB of dynamic LDS must be granted per kernel (once per device).
   static unsigned long long configured = 0;
   int dev = 0;
@@ -369,25 +425,48 @@ hipError_t launch_sk_t(const FwdArgs& a, hipStream_t stream) {
     if (e != hipSuccess) return e;
     if (dev < 64) __atomic_fetch_or(&configured, 1ull << dev, __ATOMIC_RELEASE);
   }
-  hipLaunchKernelGGL((fwd_sk_kernel<T, CAUSAL, D, FQ, NW>), dim3((unsigned)blocks), dim3(NW * kWave),
+  hipLaunchKernelGGL((fwd_sk_kernel<T, CAUSAL, D, FQ, RS, NW>), dim3((unsigned)blocks), dim3(NW * kWave),
                      lds, stream, a);
   return hipGetLastError();
 }
 
-template <typename T, bool CAUSAL, int D, bool FQ>
+// Two row sets per workgroup: a row costs about 0.8 of what it costs with one, but the units of work
+// are twice as large.  Compared is the time of the fullest CU in workgroups times keys: the longest
+// workgroup's, or the CU's share of the average one; with one set and more workgroups than CUs some
+// CU holds two of them at once.  us, fp16, d 128, one set / two: 32/8 heads, 512 rows 9.6 / 11.0, 1024
+// rows 22.1 / 18.6, 2048 rows 60.5 / 49.6; 28/4, 1531 rows 36.7 / 30.6; 12/2, 1792 rows 22.3 / 25.3,
+// 2560 rows 36.2 / 34.9, 1000 rows behind 2500 32.9 / 31.7 (bf16 37.4 / 33.5).
+template <bool CAUSAL>
+bool sk_two_sets(const FwdArgs& a) {
+  const long longest = CAUSAL ? a.start_pos + (long)a.n_q : 1;
+  const long average2 = CAUSAL ? 2l * a.start_pos + a.n_q : 2;  // twice the average
+  const long b1 = sk_blocks<CAUSAL>(a, 32), b2 = sk_blocks<CAUSAL>(a, 64), cu = a.n_cu;
+  const long one = b1 <= cu ? 2 * longest * cu : std::max(2 * cu, b1) * average2;
+  const long two = std::max(2 * longest * cu, b2 * average2);
+  return 8 * two < 5 * one;
+}
+
+template <typename T, bool CAUSAL, int D, bool FQ, int RS>
 hipError_t launch_sk_w(const FwdArgs& a, hipStream_t stream) {
   // 8 waves where a workgroup has a CU of its own anyway and keys enough for them.
   const int keys = CAUSAL ? a.start_pos + a.n_q : a.max_seqlen;
   // 32/8 heads, 256 rows behind 4000 keys: 32.2 us with 4 waves, 28.6 with 8; 137 rows 5.9 and 6.8.
-  return sk_blocks<CAUSAL>(a) <= a.n_cu && keys >= 512 ? launch_sk_t<T, CAUSAL, D, FQ, 8>(a, stream)
-                                                       : launch_sk_t<T, CAUSAL, D, FQ, 4>(a, stream);
+  return sk_blocks<CAUSAL>(a, 32 * RS) <= a.n_cu && keys >= 512
+             ? launch_sk_t<T, CAUSAL, D, FQ, RS, 8>(a, stream)
+             : launch_sk_t<T, CAUSAL, D, FQ, RS, 4>(a, stream);
+}
+
+template <typename T, bool CAUSAL, int D, bool FQ>
+hipError_t launch_sk_r(const FwdArgs& a, hipStream_t stream) {
+  return sk_two_sets<CAUSAL>(a) ? launch_sk_w<T, CAUSAL, D, FQ, 2>(a, stream)
+                                : launch_sk_w<T, CAUSAL, D, FQ, 1>(a, stream);
 }
 
 template <typename T, bool CAUSAL, int D>
 hipError_t launch_sk_d(const FwdArgs& a, hipStream_t stream) {
   if constexpr (CAUSAL && (D == 64 || D == 128))
-    if (a.rope_sin) return launch_sk_w<T, CAUSAL, D, true>(a, stream);
-  return launch_sk_w<T, CAUSAL, D, false>(a, stream);
+    if (a.rope_sin) return launch_sk_r<T, CAUSAL, D, true>(a, stream);
+  return launch_sk_r<T, CAUSAL, D, false>(a, stream);
 }
 
 template <typename T, bool CAUSAL>
@@ -407,11 +486,11 @@ hipError_t launch_sk(const FwdArgs& a, hipStream_t stream) {
 // Which launches run here, against what they ran on before: the ping-pong kernel (256-query
 // workgroups fill the device, or a key split and its merge), else the tile kernel of fwd.hip.
 // us, fp16, d 128 unless noted:
-//   causal 32/8 heads: 137 rows 8.2 -> 5.9, 512 rows 22.9 -> 9.7, 1536 rows 41.3 -> 38.4, 2048 rows
-//   57.7 against 60.1; 12/2: 2048 rows 32.6 -> 25.7, 3072 rows 53.2 -> 49.3, 1024 rows behind 3000
-//   36.4 against 36.9; 28/4 (tile kernel before): 2048 rows 68.6 -> 55.0
-//   vision, 16 heads, d 72: one image of 1024 26.7 -> 13.3, of 2300 (tile kernel) 67.8 -> 48.2;
-//   four of 1024 (fill the device) 30.3 against 40.3
+//   causal 32/8 heads: 137 rows 8.2 -> 5.7, 512 rows 23.1 -> 9.6, 1531 rows 42.0 -> 33.1, 2560 rows
+//   74.2 -> 73.0, 3072 rows 90.8 against 96.6; 28/4: 1531 rows 40.4 -> 30.6 (bf16 41.2 -> 31.6); 12/2:
+//   2560 rows 43.1 -> 34.9, 1000 rows behind 2500 34.1 -> 31.7 (bf16 38.2 -> 33.5)
+//   vision, 16 heads, d 72: one image of 1024 27.2 -> 12.7, of 2300 (tile kernel) 67.7 -> 53.0;
+//   four of 1024 (fill the device) 30.5 against 36.9
 bool fwd_sk_prefers(const FwdArgs& a, int dtype, bool causal) {
   if (!fwd_pp_supports(a, dtype)) return false;
   const long n_q = causal ? a.n_q : a.max_seqlen;
@@ -419,21 +498,29 @@ bool fwd_sk_prefers(const FwdArgs& a, int dtype, bool causal) {
   if (n_q * a.kv_mul >= (1l << 30)) return false;  // packed rows are ints
   // One or two key tiles: the merge costs more than the split saves (24 rows 5.0 against 5.4).
   if (keys <= 64) return false;
-  const long blocks = causal ? sk_blocks<true>(a) : sk_blocks<false>(a);
+  const long blocks = causal ? sk_blocks<true>(a, 32) : sk_blocks<false>(a, 32);
   // Many short segments already fill the device (8 of 256: 10.6 against 11.3).
   if (!causal && keys <= 256 && blocks > 2l * a.n_cu) return false;
-  size_t bytes;
-  const bool key_split = causal && fwd_pp_key_split(a, dtype, a.n_cu, &bytes) > 0;
-  const long pp_blocks = (causal ? 1 : a.n_seg) * ((n_q + 255) / 256) * a.Hq;
-  if (!key_split && pp_blocks < 256) return true;  // the tile kernel would run
-  // Few rows behind a long prefix: a workgroup's own chain is the longer one (12/2 heads, 128 rows
-  // behind 6000 28.0 against 29.4; 28/4 heads, 112 workgroups, 31.8 against 30.1).
-  if (key_split && blocks * 4 < a.n_cu && keys > 4096) return false;
-  // Wave tiles (32 rows x 32 keys) in all, each 16 KB through a CU's L2 path (10 KB at head size
-  // 64); for segments an upper bound, since the host does not know their lengths.
+  // Wave tiles (32 rows x 32 keys) in all; for segments an upper bound, since the host does not know
+  // their lengths.
   const long tiles = causal ? blocks * (2l * a.start_pos + a.n_q) / 64
                             : ((long)a.n_q * a.kv_mul + 31) / 32 * a.Hkv * ((keys + 31) / 32);
-  return tiles * (causal && a.head_size == 64 ? 5 : 8) <= 1280l * a.n_cu;
+  const bool causal_fits = causal && tiles * (a.head_size == 64 ? 5 : 8) <= 3200l * a.n_cu;
+  if (causal_fits && keys <= 4096) return true;  // whatever the key split would be
+  size_t bytes;
+  const long chunk = causal ? fwd_pp_key_split(a, dtype, a.n_cu, &bytes) : 0;
+  const long pp_blocks = (causal ? 1 : a.n_seg) * ((n_q + 255) / 256) * a.Hq;
+  if (chunk == 0 && pp_blocks < 256) return true;  // the tile kernel would run
+  // Few rows behind a long prefix: a workgroup's own chain is the longer one (12/2 heads, 128 rows
+  // behind 6000 28.0 against 29.4; 28/4 heads, 112 workgroups, 31.8 against 30.1).
+  if (chunk > 0 && blocks * 4 < a.n_cu && keys > 4096) return false;
+  if (!causal) return tiles * 8 <= 1280l * a.n_cu;
+  // A key split whose chunks cover 84 % of the device, behind a long prefix (700 rows behind 3500: 28/4
+  // heads 53.6 against 61.7, 12/2 32.0 against 34.1; 512 behind 6000, 28/4, 82 %, 60.2 against 57.5).
+  if (chunk > 0 && a.start_pos >= a.n_q && keys > 4096 &&
+      pp_blocks * (2l * a.start_pos + a.n_q) * 100 > 84 * 128 * chunk * a.n_cu)
+    return false;
+  return causal_fits;
 }
 
 hipError_t launch_fwd_sk(const FwdArgs& a, int dtype, bool causal, hipStream_t stream) {

@@ -1,5 +1,5 @@
-"""Attention whose keys are split inside the workgroup (fwd_sk.hip): 32-row tiles of packed query
-heads, 32-key tiles over 4 or 8 waves.  Shapes sit at the edges of those tiles and of the dispatch
+"""Attention whose keys are split inside the workgroup (fwd_sk.hip): tiles of 32 or 64 packed
+query rows, 32-key tiles over 4 or 8 waves.  Shapes sit at the edges of those tiles and of the dispatch
 (up to 64 keys, and launches that fill the device, run elsewhere)."""
 import numpy as np
 import pytest
@@ -60,7 +60,41 @@ def test_sk_varlen_segments(kind, d, cu):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["fp16", "bf16"])
-@pytest.mark.parametrize("Hq,Hkv,d,start,S", [(28, 4, 128, 0, 700), (6, 2, 64, 500, 90)])
+@pytest.mark.parametrize("d", [64, 72, 80, 96, 128])
+@pytest.mark.parametrize("Hq,Hkv,start,S", [(16, 16, 0, 1501), (9, 3, 2600, 1333), (32, 8, 190, 290)])
+def test_sk_causal_two_row_sets(kind, d, Hq, Hkv, start, S):
+    """64 rows per workgroup (grids of more than two workgroups of 32 rows per CU, or that little
+    above one): last workgroups with one set, or part of one, in range; 4 and 8 waves."""
+    rng = np.random.default_rng(9400 + d + S)
+    q, kc, vc, out = run_prefill(kind, start, S, Hq, Hkv, d, start + S, 1, 0, rng)
+    rows = np.unique(np.concatenate([sample_rows(S, 20, rng), [0, 31, 32, 63, 64, S - 2, S - 1]]))
+    ref = oracle.prefill_causal(start, q, kc, vc, Hq, Hkv, d, rows=rows, nthreads=8)
+    assert_lowp_close(out[rows], ref, what=f"{kind} d {d} S {S} start {start}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("d", [64, 72, 80, 96, 128])
+@pytest.mark.parametrize("cu", [(0, 1000, 1001, 1700), (0, 1473)])
+def test_sk_varlen_two_row_sets(kind, d, cu):
+    rng = np.random.default_rng(9500 + d + cu[-1])
+    H, N = 16, cu[-1]
+    q, k, v = vision_inputs(rng, np.array(cu, np.int32), H, d, kind)
+    out = torch.zeros(N, H * d, device="cuda", dtype=TORCH[kind])
+    K.vision_attention_varlen_cu(dev(q, kind), dev(k, kind), dev(v, kind), out,
+                                 torch.tensor(cu, dtype=torch.int32, device="cuda"),
+                                 int(np.diff(cu).max()), H, d)
+    torch.cuda.synchronize()
+    rows = np.unique(np.concatenate([[c for c in cu if c < N], np.array(cu[1:]) - 1, [31, 32, 63, 64],
+                                     rng.integers(0, N, 16)]))
+    ref = oracle.varlen_bidir(q, k, v, np.array(cu, np.int32), rows=rows, nthreads=8)
+    assert_lowp_close(out.float().cpu().numpy()[rows], ref, what=f"{kind} d {d} {cu}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("Hq,Hkv,d,start,S", [(28, 4, 128, 0, 700), (6, 2, 64, 500, 90), (28, 4, 128, 0, 1110),
+                                              (16, 16, 64, 0, 1501), (12, 2, 128, 2500, 1000)])
 def test_sk_fused_q_and_aliased_output(kind, Hq, Hkv, d, start, S):
     """The fused Q producer gives the bits of the producer followed by the prefill, and the
     output may be the query."""
